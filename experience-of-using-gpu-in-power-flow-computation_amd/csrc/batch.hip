@@ -1242,7 +1242,12 @@ namespace {
         pf_status s_ = (expr);      \
         if (s_ != PF_OK) return s_; \
     } while (0)
-constexpr long long kLdsLimit = 64 * 1024;
+// Largest working set held in LDS (MODE 2): two workgroups of it, with the
+// kernel's static LDS, share the 160 KiB of a CU.  118 buses in FP64 take
+// 71 KiB: 333 scenarios 411 us there, 475 us at the best MODE 1 shape.  A
+// set that leaves one workgroup per CU gains nothing: 236 buses in FP32
+// (80 KiB) 1,740 us in LDS, 1,140 us in MODE 1.
+constexpr long long kLdsLimit = 75 * 1024;
 }  // namespace
 
 namespace {
@@ -1332,6 +1337,7 @@ struct pf_batch {
     pf_status launch_all();
     pf_status configure(BatchNet &nb, int mode, int block, int per_cu);
     pf_status occupancy(const BatchNet &nb, int mode, int block, int *per_cu);
+    pf_status default_shape(const BatchNet &nb, int nscen, int *block, int *per_cu);
     void drop_graph() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
@@ -1471,6 +1477,10 @@ pf_status pf_batch::add_net(const pf_network &src) {
     b->ws = mixed ? work_bytes<float>(nB, n, net.nPV, sym.nblk())
                   : work_bytes<double>(nB, n, net.nPV, sym.nblk());
     b->lds = b->ws <= kLdsLimit;
+    if (b->lds)
+        for (int blk : {256, 512, 1024})
+            BHIP(hipFuncSetAttribute((const void *)batch_kernel(mixed, 2, blk),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit));
     b->block = b->lds ? 256 : 1024;
     if (b->lds) {
         b->mode = 2;
@@ -1506,6 +1516,43 @@ pf_status pf_batch::occupancy(const BatchNet &nb, int mode, int block, int *per_
     BHIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc, (const void *)batch_kernel(mixed, mode, block), block,
                                                       shm));
     *per_cu = pc;
+    return PF_OK;
+}
+
+// The launch shape of nscen scenarios when none was chosen.  A scenario alone
+// on its CU is fastest in a wide workgroup; with more scenarios than CUs it
+// pays to keep several narrow ones resident, whose barriers and loads
+// overlap, as long as they fit (118 buses, FP64: 24 scenarios 320 us at 512
+// threads, 373 at 256; 333 scenarios 601 at 512 and one per CU, 411 at 256
+// and two per CU).
+//   LDS (MODE 2): 512 threads up to one scenario per CU, 256 above; up to 64
+//   nodes and more scenarios than fit at once, 128 (57 buses, FP32, 1,500
+//   scenarios: 463 -> 339 us).
+//   MODE 1 / 0: 1024 threads, one per CU; up to kNarrowNodes nodes and more
+//   scenarios than CUs, two of 256 (354 buses, FP64, 1,500 scenarios: 6.11
+//   -> 4.51 ms; on 590 buses 15.8 -> 18.9, so not there).
+constexpr int kNarrowNodes = 400;
+pf_status pf_batch::default_shape(const BatchNet &nb, int nscen, int *block, int *per_cu) {
+    int occ = 0;
+    if (nb.mode == 2) {
+        *block = nscen <= cus ? 512 : 256;
+        BCHK(occupancy(nb, 2, *block, &occ));
+        if (nscen > occ * cus && nscen > cus && nb.sym.n <= 64) {
+            *block = 128;
+            BCHK(occupancy(nb, 2, *block, &occ));
+        }
+        *per_cu = occ;
+        return PF_OK;
+    }
+    *block = 1024;
+    *per_cu = 1;
+    if (nscen > cus && nb.sym.n <= kNarrowNodes) {
+        BCHK(occupancy(nb, nb.mode, 256, &occ));
+        if (occ >= 2) {
+            *block = 256;
+            *per_cu = 2;
+        }
+    }
     return PF_OK;
 }
 
@@ -1715,9 +1762,10 @@ pf_status pf_batch_set_scenarios(pf_batch *b, int n_scen, const int *net_of, con
             BatchNet &nb = *nbp;
             if (nb.scen.empty()) continue;
             BCHK(b->upload(&nb.d_scen, nb.scen));
-            // default shape: as many resident workgroups as fit for LDS
-            // topologies, one per CU otherwise (pf_batch_autotune refines it)
-            BCHK(b->configure(nb, nb.mode, nb.block, nb.lds ? 0 : 1));
+            // default shape from the scenario count (pf_batch_autotune refines it)
+            int block = 0, per_cu = 0;
+            BCHK(b->default_shape(nb, (int)nb.scen.size(), &block, &per_cu));
+            BCHK(b->configure(nb, nb.mode, block, per_cu));
         }
     }
     const size_t tot = (size_t)b->total;
@@ -1962,13 +2010,13 @@ extern "C" pf_status pf_batch_solve_noalloc(pf_batch *b, int n_scen, const int *
     int n_big = 0;
     for (auto &nb : b->nets) n_big += nb->mode != 2;
     const long long share = n_big ? (kScratchBytes - o_ws) / n_big : 0;
-    struct Plan { int grid; long long ws_off; };
+    struct Plan { int grid, block; long long ws_off; };
     Plan plan[64];            // at most 64 networks per batch (pf_batch_create)
     long long o = o_ws;
     for (int i = 0; i < nn; i++) {
         BatchNet &nb = *b->nets[i];
-        int per_cu = nb.per_cu;
-        if (nb.grid == 0) BCHK(b->occupancy(nb, nb.mode, nb.block, &per_cu));
+        int block = nb.block, per_cu = nb.per_cu;
+        if (nb.grid == 0) BCHK(b->default_shape(nb, n_scen, &block, &per_cu));
         int grid = std::max(1, per_cu * b->cus);
         if (nb.mode != 2) {
             grid = (int)std::min<long long>(grid, share / nb.ws);
@@ -1977,7 +2025,7 @@ extern "C" pf_status pf_batch_solve_noalloc(pf_batch *b, int n_scen, const int *
                 return PF_INVALID_ARG;
             }
         }
-        plan[i] = {grid, o};
+        plan[i] = {grid, block, o};
         if (nb.mode != 2) o += up((long long)grid * nb.ws);
     }
     if (o > kScratchBytes) {
@@ -2019,8 +2067,8 @@ extern "C" pf_status pf_batch_solve_noalloc(pf_batch *b, int n_scen, const int *
         J.diverge = 1e6;
         BatchTopo tp = nb.tp;
         void *args[] = {&tp, &J};
-        BHIP(hipLaunchKernel((const void *)batch_kernel(mixed, nb.mode, nb.block), dim3(plan[i].grid),
-                             dim3(nb.block), args, nb.mode == 0 ? 0 : (size_t)nb.shm, s));
+        BHIP(hipLaunchKernel((const void *)batch_kernel(mixed, nb.mode, plan[i].block), dim3(plan[i].grid),
+                             dim3(plan[i].block), args, nb.mode == 0 ? 0 : (size_t)nb.shm, s));
     }
     if (!stream) {
         BHIP(hipStreamSynchronize(s));
