@@ -195,7 +195,7 @@ pf_status pf_probe_flat_factor_solve(const pf_symbolic_probe *p, double *blocks,
     std::memcpy(b.data(), blocks, sizeof(double) * 4 * (size_t)s.nslot());
     pf::FlatTail parts, top;
     if (s.n_parts > 0) parts = pf::flat_parts(s);
-    if (s.tail_start < s.nlev_s) top = pf::flat_tail(s, s.tail_start, true);
+    if (s.tail_start < s.nlev_s) top = pf::flat_tail(s, s.tail_start, true, std::max(64, s.n));
     if (!pf::host_flat_factor(s, parts, top, b.data())) return PF_SINGULAR;
     pf::PartSweeps ps;
     if (s.n_parts > 0) ps = pf::part_sweeps(s);

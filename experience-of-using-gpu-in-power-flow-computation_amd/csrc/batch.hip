@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cstdio>
 #include <cstring>
 #include <memory>
@@ -944,7 +945,7 @@ __device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Wo
             for (int l = 0; l < Y.nlev_s;) {
                 if (s_ck && tp.F.fl_ptr && l == tp.F.lv0 && ((size_t)w.x & 15) == 0) {   // flat pair lists
                     T *pa = reinterpret_cast<T *>(w.x);   // x and r: free until the solve
-                    flat_factor_levels<T, 1>(Y, tp.F, w.blk, 0, Y.nlev_s - tp.F.lv0, &s_sing, pa,
+                    flat_factor_levels<T, 1>(Y, tp.F, w.blk, 0, tp.F.nsteps, &s_sing, pa,
                                                 pa + 4 * (size_t)tp.F.max_pairs);
                     break;
                 }
@@ -1361,7 +1362,7 @@ pf_status pf_batch::add_net(const pf_network &src) {
         const long long w0 = mx ? work_bytes<float>(src.nB, b->sym.n, src.nPV, b->sym.nblk())
                                 : work_bytes<double>(src.nB, b->sym.n, src.nPV, b->sym.nblk());
         if (w0 > kLdsLimit && opt.lu_blocked)
-            b->sym = analyze(src, b->yp, kWideLevel - 1, kBatchChainWide, kTopWidth);
+            dense_top(b->sym, kBatchChainWide, kTopWidth);
     }
     chunk_tail(b->sym, kBatchChunkPairs);
     if (!b->sym.level_ordered()) {
@@ -1433,18 +1434,25 @@ pf_status pf_batch::add_net(const pf_network &src) {
     }
     // the factorisation as flat pair lists, its products in the step vectors
     // x and r (4 n doubles, free during the factorisation): from the first
-    // level when one level's products fit there, else from the narrow top
+    // level, wide levels cut into steps whose products fit there, unless
+    // that takes over half as many steps again as there are levels (a step
+    // costs two barriers and a round of loads), else from the narrow top,
+    // uncut.  1,888 buses in FP32, 38 steps for 33 levels, 100 scenarios:
+    // 2,040 us; level by level below the top 2,360
     b->tp.F = DevFlat{};
     if (opt.lu_blocked && sym.tail_start < sym.nlev_s) {
         const bool mx = opt.precision != PF_FP64;
         auto need = [&](const FlatTail &f) {
             return mx ? flat_tail_lds<float>(f.max_pairs, f.max_col) : flat_tail_lds<double>(f.max_pairs, f.max_col);
         };
-        FlatTail ft = flat_tail(sym, 0, false);
-        if (need(ft) > 32LL * sym.n) ft = flat_tail(sym, sym.tail_start, false);
+        const int step_blocks = (int)(32LL * sym.n / (mx ? 16 : 32));
+        FlatTail ft = flat_tail(sym, 0, false, step_blocks);
+        if (need(ft) > 32LL * sym.n || 2 * ft.fl_ptr.size() > 3 * (size_t)sym.nlev_s + 2)
+            ft = flat_tail(sym, sym.tail_start, false, INT_MAX);
         if (need(ft) <= 32LL * sym.n) {
             DevFlat &F = b->tp.F;
             F.lv0 = ft.lv0;
+            F.nsteps = (int)ft.fl_ptr.size() - 1;
             F.max_pairs = ft.max_pairs;
             F.max_col = ft.max_col;
             F.de_sentinel = ft.de_ptr.back();

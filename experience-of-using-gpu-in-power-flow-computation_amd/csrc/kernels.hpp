@@ -119,7 +119,7 @@ struct DevTail {
 // [fl_ptr[t], fl_ptr[t+1]) (fl_s: a pair's staged slots in the previous
 // step, or -1); lv0: the first level of a level-by-level program.
 struct DevFlat {
-    int lv0, max_pairs, max_col, de_sentinel;
+    int lv0, nsteps, max_pairs, max_col, de_sentinel;
     const int *fl_ptr, *fl_split, *fl_a, *fl_b, *fl_s, *de_ptr;
     const int *de_node, *de_p, *de_q0, *de_ext, *de_lo, *de_hi, *de_dlo, *de_dhi, *de_lr, *st_g;
 };

@@ -123,6 +123,9 @@ struct Symbolic {
 // top_width: widest elimination-tree level it may take
 Symbolic analyze(const pf_network &net, const YPattern &yp, int tail_width, int chain_cap, int top_width);
 
+// chooses the dense top of an analysed network anew
+void dense_top(Symbolic &s, int chain_cap, int top_width);
+
 constexpr int kChunkPairs = 16;
 constexpr int kChunkDiag = 1 << 30, kChunkMask = kChunkDiag - 1;
 // Builds the chunk lists of the tail levels [tail_start, nlev_s), chunks of
@@ -169,8 +172,10 @@ TailSweeps tail_sweeps(const Symbolic &s);
 // pair and destination lists end with one sentinel entry past the program
 // (pair 0; a pivot of node 0 without pairs), which lanes without a pair or
 // a destination read when they prefetch; de_ptr.back() is its index.
-//   flat_tail: levels [lv0, nlev_s), step t = level lv0 + t, destinations
-//   in ld order; with split_below (single-network solver, lv0 = tail_start)
+//   flat_tail: levels [lv0, nlev_s) in order, destinations in ld order; a
+//   level of more than step_blocks products (a node's own aside) is cut
+//   into several steps of whole nodes, so that a step's products fit the
+//   memory a kernel has for them.  With split_below (single-network solver, lv0 = tail_start)
 //   the pairs from sources below lv0 (k < lvl_ptr[lv0]) are left to a
 //   grid-wide pass, without it (one workgroup per scenario) the lists hold
 //   every pair.
@@ -183,7 +188,7 @@ struct FlatTail {
     int max_pairs = 0, max_col = 0;
     bool stage_ok = true;   // fl_s is usable (a pair's two positions always share a step)
 };
-FlatTail flat_tail(const Symbolic &s, int lv0, bool split_below);
+FlatTail flat_tail(const Symbolic &s, int lv0, bool split_below, int step_blocks);
 FlatTail flat_parts(const Symbolic &s);
 // Starting state of every scenario of a batch from rows of an array on GPU
 // `device` (row s: scenario s; |V| = row[v_col + i] * sd[v_col + i] +

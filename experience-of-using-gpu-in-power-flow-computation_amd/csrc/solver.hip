@@ -437,6 +437,7 @@ pf_status pf_solver::setup_tail_sweeps() {
 // the LDS holds one level's products.
 pf_status pf_solver::upload_flat(const FlatTail &ft, DevFlat &F) {
     F.lv0 = ft.lv0;
+    F.nsteps = (int)ft.fl_ptr.size() - 1;
     F.max_pairs = ft.max_pairs;
     F.max_col = ft.max_col;
     F.de_sentinel = ft.de_ptr.back();
@@ -471,7 +472,7 @@ pf_status pf_solver::setup_flat_tail() {
         out = (int)bytes;
         return PF_OK;
     };
-    const FlatTail ft = flat_tail(sym, sym.tail_start, true);
+    const FlatTail ft = flat_tail(sym, sym.tail_start, true, (int)(cap / (opt.precision == PF_MIXED ? 24 : 32)));
     flat_ne = ft.de_ptr.back();
     PFCHK(upload_flat(ft, dfl));
     PFCHK(allow((const void *)k_factor_tail_flat<double>,
@@ -537,7 +538,7 @@ pf_status pf_solver::enqueue_lu(T *blk, int gate) {
     const int fl = sym.tail_start < sym.nlev_s ? flat_lds[sizeof(T) == 4 ? 1 : 0] : 0;
     if (fl) {   // narrow levels below the chain: pairs from below the tail across the GPU first
         k_tail_factor_ext<T><<<(flat_ne + 31) / 32, 256, 0, stream>>>(dy, dfl, blk, ctl, flat_ne, gate);
-        k_factor_tail_flat<T><<<1, 1024, fl, stream>>>(dy, dfl, blk, ctl, sym.nlev_s - sym.tail_start, gate,
+        k_factor_tail_flat<T><<<1, 1024, fl, stream>>>(dy, dfl, blk, ctl, dfl.nsteps, gate,
                                                        sizeof(T) == 4 ? flat_cap : 0);
     } else if (sym.tail_start < sym.nlev_s) {
         k_factor_tail<T><<<1, 1024, 0, stream>>>(dy, blk, ctl, sym.tail_start, sym.nlev_s, gate);
