@@ -9,7 +9,6 @@
 //   k_factor_*,
 //   k_fwd_*/k_bwd_* cusolverSpDcsrlsvqr, GPU/newtonRaphson.cuh:466-468
 //   k_update        attOlim / attVlim, GPU/newtonRaphson.cuh:76-119
-//   k_dense         cusolverDnDgetrf/getrs, GPU/newtonRaphson.cuh:507-530
 #include "kernels_impl.hpp"
 
 namespace pf {
@@ -1045,8 +1044,7 @@ __global__ void __launch_bounds__(256) k_update(DevNet N, DevState S, int gate) 
 
 // ------------------------------------------------------------ dense path
 // metodo denso: the block Jacobian scattered into a dense column-major
-// matrix (node order, 2n x 2n) and factored by one workgroup with partial
-// pivoting; the right-hand side is eliminated alongside.
+// matrix (node order, 2n x 2n), factored by the kernels of dense.hip.
 __global__ void k_dense_scatter(DevSym Y, const double *blk, double *A, int ld, Ctl *ctl, int gate) {
     if (gate && !ctl->step) return;
     int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1068,69 +1066,6 @@ __global__ void k_dense_scatter(DevSym Y, const double *blk, double *A, int ld, 
     A[(size_t)(2 * c + 1) * ld + 2 * r] = v.b;
     A[(size_t)(2 * c) * ld + 2 * r + 1] = v.c;
     A[(size_t)(2 * c + 1) * ld + 2 * r + 1] = v.d;
-}
-
-__global__ void __launch_bounds__(1024) k_dense(double *A, double *b, int n, Ctl *ctl, int gate) {
-    if (gate && !ctl->step) return;
-    __shared__ double sv[16];
-    __shared__ int si[16];
-    __shared__ int s_piv;
-    const int tid = threadIdx.x, w = tid / 64, lane = tid & 63;
-    for (int k = 0; k < n; k++) {
-        double best = -1.0;
-        int bi = k;
-        for (int i = k + tid; i < n; i += 1024) {
-            double a = fabs(A[(size_t)k * n + i]);
-            if (a > best) { best = a; bi = i; }
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            double ob = __shfl_xor(best, off);
-            int oi = __shfl_xor(bi, off);
-            if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
-        }
-        if (lane == 0) { sv[w] = best; si[w] = bi; }
-        __syncthreads();
-        if (tid == 0) {
-            double bb = sv[0];
-            int ii = si[0];
-            for (int q = 1; q < 16; q++)
-                if (sv[q] > bb || (sv[q] == bb && si[q] < ii)) { bb = sv[q]; ii = si[q]; }
-            s_piv = (bb > 0.0 && isfinite(bb)) ? ii : -1;
-        }
-        __syncthreads();
-        const int p = s_piv;
-        if (p < 0) {
-            if (tid == 0) atomicOr(&ctl->singular, 1);
-            return;   // uniform: every thread read the same s_piv
-        }
-        if (p != k) {
-            for (int c = tid; c < n; c += 1024) {
-                double t = A[(size_t)c * n + k];
-                A[(size_t)c * n + k] = A[(size_t)c * n + p];
-                A[(size_t)c * n + p] = t;
-            }
-            if (tid == 0) { double t = b[k]; b[k] = b[p]; b[p] = t; }
-        }
-        __syncthreads();
-        const double piv = A[(size_t)k * n + k];
-        for (int i = k + 1 + tid; i < n; i += 1024) A[(size_t)k * n + i] /= piv;
-        __syncthreads();
-        const double bk = b[k];
-        for (int i = k + 1 + tid; i < n; i += 1024) {
-            const double li = A[(size_t)k * n + i];
-            for (int c = k + 1; c < n; c++) A[(size_t)c * n + i] -= li * A[(size_t)c * n + k];
-            b[i] -= li * bk;
-        }
-        __syncthreads();
-    }
-    for (int k = n - 1; k >= 0; k--) {
-        if (tid == 0) b[k] /= A[(size_t)k * n + k];
-        __syncthreads();
-        const double bk = b[k];
-        for (int i = tid; i < k; i += 1024) b[i] -= A[(size_t)k * n + i] * bk;
-        __syncthreads();
-    }
 }
 
 // explicit instantiations

@@ -41,6 +41,5 @@ __global__ void k_fill(double *x, size_t n, double v);
 template <int LPR> __global__ void k_residual(DevNet N, DevState S, int gate);
 __global__ void k_update(DevNet N, DevState S, int gate);
 __global__ void k_dense_scatter(DevSym Y, const double *blk, double *A, int ld, Ctl *ctl, int gate);
-__global__ void k_dense(double *A, double *b, int n, Ctl *ctl, int gate);
 
 }  // namespace pf

@@ -20,6 +20,7 @@
 #include <string>
 #include <vector>
 
+#include "dense.hpp"
 #include "kernels_decl.hpp"
 #include "pf_internal.hpp"
 
@@ -78,6 +79,7 @@ struct pf_solver {
     double *blk64 = nullptr;
     float *blk32 = nullptr;
     double *dense = nullptr;
+    int *dense_chg = nullptr;   // the dense panel's row swaps
     Ctl *ctl = nullptr;
     Ctl *ctl_host = nullptr;      // pinned, 2 slots
     hipGraph_t graph = nullptr;
@@ -326,7 +328,8 @@ pf_status pf_solver::build() {
 pf_status pf_solver::ensure_dense() {
     if (dense) return PF_OK;
     size_t m = 2 * (size_t)sym.n;
-    if (m > 4096) return PF_INVALID_ARG;   // dense path is for systems up to 4096 unknowns
+    if (m > kDenseMax) return PF_INVALID_ARG;
+    PFCHK(alloc(&dense_chg, kDenseSwaps));
     return alloc(&dense, m * m);
 }
 
@@ -606,7 +609,7 @@ pf_status pf_solver::enqueue_factor_solve(int gate) {
         k_fill<<<(unsigned)((mm + 255) / 256), 256, 0, stream>>>(dense, mm, 0.0);
         k_dense_scatter<<<(sym.nslot() + 255) / 256, 256, 0, stream>>>(dy, blk64, dense, m, ctl, gate);
         k_copy<<<(m + 255) / 256, 256, 0, stream>>>(ds.x, ds.g, m, ctl, gate);
-        k_dense<<<1, 1024, 0, stream>>>(dense, ds.x, m, ctl, gate);
+        launch_dense_solve(dense, ds.x, m, dense_chg, ctl, gate, stream);
     } else if (mixed()) {
         PFCHK(enqueue_lu(blk32, gate));
         k_copy<<<(m + 255) / 256, 256, 0, stream>>>(ds.x, ds.g, m, ctl, gate);

@@ -345,3 +345,40 @@ def test_nr_traced_limits(pf, oracle, variant):
     assert r["n_switch_events"] == o["n_switch_events"] == 2
     assert np.array_equal(lq, o["limQ"])
     assert np.abs(V - o["V"]).max() <= 1e-9 and np.abs(th - o["theta"]).max() <= 1e-9
+
+
+@pytest.mark.parametrize("name", ["ieee14", "ieee30", "ieee57", "c118", "c944"])
+def test_dense_lu_solve(pf, oracle, cases, name):
+    """metodo denso's LU at unknown counts around its panels of 32 columns (26
+    to 234) and in its panels of 8 (1,886), whose rows sit four per thread:
+    backward error within n times the rounding unit times the growth that
+    partial pivoting shows in practice."""
+    p = _path(cases, name)
+    _say("dense lu_solve", name)
+    net = pf.Network(p)
+    s = _solver(pf, net, metodo=pf.DENSO)
+    oc = oracle.Case(p)
+    rp, ci, y = oc.ybus()
+    V = 1.0 + 0.01 * np.random.default_rng(1).standard_normal(net.nB)
+    th = 0.05 * np.random.default_rng(2).standard_normal(net.nB)
+    lq = _limq(net, 3)
+    Po, Qo = oracle.pq(rp, ci, y, V, th)
+    pqlim = np.sort(np.concatenate([net.pq, net.pv[lq]]))
+    rpo, co, vo = oracle.jacobian(net.nB, net.slack, rp, ci, y, V, th, Po, Qo, pqlim)
+    n = len(rpo) - 1
+    J = csr_to_dense(rpo, co, vo, n)
+    b = np.random.default_rng(4).standard_normal(n)
+    x = s.lu_solve(V, th, lq, b)
+    r = np.abs(J @ x - b).max()
+    assert r <= 10 * n * 2.0 ** -53 * (np.abs(J).sum(1).max() * np.abs(x).max() + np.abs(b).max())
+
+
+def test_dense_lu_singular(pf, cases):
+    """A column without a finite pivot ends the dense solve as singular."""
+    net = pf.Network(_path(cases, "c118"))
+    s = _solver(pf, net, metodo=pf.DENSO)
+    V = np.ones(net.nB)
+    V[net.pq[3]] = np.nan
+    with pytest.raises(pf.PfError) as e:
+        s.lu_solve(V, np.zeros(net.nB), None, np.ones(net.nB - 1 + net.nPQ))
+    assert e.value.status == pf.PF_SINGULAR
