@@ -1280,6 +1280,7 @@ struct BatchNet {
     int block = 256;
     int grid = 0;
     int per_cu = 1;            // workgroups per CU the grid is sized for
+    int occ[3][17] = {};       // workgroups per CU by mode and block / 64, 0: not asked for yet
     long long ws = 0;
     std::vector<int> scen;
     // device
@@ -1337,8 +1338,8 @@ struct pf_batch {
     pf_status launch_net(size_t i, hipStream_t s);
     pf_status launch_all();
     pf_status configure(BatchNet &nb, int mode, int block, int per_cu);
-    pf_status occupancy(const BatchNet &nb, int mode, int block, int *per_cu);
-    pf_status default_shape(const BatchNet &nb, int nscen, int *block, int *per_cu);
+    pf_status occupancy(BatchNet &nb, int mode, int block, int *per_cu);
+    pf_status default_shape(BatchNet &nb, int nscen, int *block, int *per_cu);
     void drop_graph() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
@@ -1356,13 +1357,13 @@ pf_status pf_batch::add_net(const pf_network &src) {
     b->yp = build_ypattern(src);
     // tail_start: the first level of the narrow top (fewer than kWideLevel
     // nodes per level up to the dense block)
-    b->sym = analyze(src, b->yp, kWideLevel - 1, opt.lu_blocked ? kBatchChain : 0, kTopWidth);
+    b->sym = analyze(src, b->yp, kWideLevel - 1, opt.lu_blocked ? kBatchChain : 0, 16);
     {   // a working set beyond LDS runs in MODE 1 / 0, whose kernels take a wider dense top
         const bool mx = opt.precision != PF_FP64;
         const long long w0 = mx ? work_bytes<float>(src.nB, b->sym.n, src.nPV, b->sym.nblk())
                                 : work_bytes<double>(src.nB, b->sym.n, src.nPV, b->sym.nblk());
         if (w0 > kLdsLimit && opt.lu_blocked)
-            dense_top(b->sym, kBatchChainWide, kTopWidth);
+            dense_top(b->sym, kBatchChainWide, 64);
     }
     chunk_tail(b->sym, kBatchChunkPairs);
     if (!b->sym.level_ordered()) {
@@ -1517,13 +1518,18 @@ pf_status pf_batch::add_net(const pf_network &src) {
 }
 
 // resident workgroups per CU of k_batch<T, mode> at this block size
-pf_status pf_batch::occupancy(const BatchNet &nb, int mode, int block, int *per_cu) {
+pf_status pf_batch::occupancy(BatchNet &nb, int mode, int block, int *per_cu) {
+    int &known = nb.occ[mode][block / 64];
+    if (known) {
+        *per_cu = known;
+        return PF_OK;
+    }
     const bool mixed = opt.precision != PF_FP64;
     const size_t shm = mode == 2 ? (size_t)nb.ws : mode == 1 ? (size_t)nb.partial : 0;
     int pc = 0;
     BHIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc, (const void *)batch_kernel(mixed, mode, block), block,
                                                       shm));
-    *per_cu = pc;
+    *per_cu = known = pc;
     return PF_OK;
 }
 
@@ -1540,7 +1546,7 @@ pf_status pf_batch::occupancy(const BatchNet &nb, int mode, int block, int *per_
 //   scenarios than CUs, two of 256 (354 buses, FP64, 1,500 scenarios: 6.11
 //   -> 4.51 ms; on 590 buses 15.8 -> 18.9, so not there).
 constexpr int kNarrowNodes = 400;
-pf_status pf_batch::default_shape(const BatchNet &nb, int nscen, int *block, int *per_cu) {
+pf_status pf_batch::default_shape(BatchNet &nb, int nscen, int *block, int *per_cu) {
     int occ = 0;
     if (nb.mode == 2) {
         *block = nscen <= cus ? 512 : 256;

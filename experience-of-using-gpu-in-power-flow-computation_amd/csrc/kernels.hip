@@ -406,12 +406,17 @@ __global__ void __launch_bounds__(256) k_chain_schur(DevSym Y, T *blk, Ctl *ctl,
 }
 
 // Gauss-Jordan inverse of the chain's Schur complement, in one workgroup (in FP32
-// with the fused update: this solver's FP32 factor is refined in FP64).
-template <typename T>
+// with the fused update: this solver's FP32 factor is refined in FP64), S in
+// TR x TC register tiles of 2x2 blocks: the smallest that 1024 threads cover
+// (chain_tile).  A step's time is its tile's arithmetic, so a chain of a few
+// nodes in the largest tiles paid for blocks it does not have: 13 nodes in
+// FP64 38 us at 4 x 3, 9 at 1 x 1; 83 nodes 279 us at 4 x 3, 225 at 3 x 3 (FP32
+// 125 us at 4 x 4, 105 at 3 x 3).
+template <typename T, int TR, int TC>
 __global__ void __launch_bounds__(ChainTiles<T>::threads) k_chain_invert(DevSym Y, T *blk, Ctl *ctl, int gate) {
     if (gate && !ctl->step) return;
     __shared__ B4<T> lds[4 * kChainMax + 2];
-    chain_invert<T, ChainTiles<T>::tr, ChainTiles<T>::tc, sizeof(T) == 4>(Y, blk, &ctl->singular, lds);
+    chain_invert<T, TR, TC, sizeof(T) == 4>(Y, blk, &ctl->singular, lds);
 }
 
 // ----------------------------------------------------- triangular solves
@@ -1083,8 +1088,14 @@ template __global__ void k_bwd_parts<double>(DevSym, const double *, double *, C
 template __global__ void k_bwd_parts<float>(DevSym, const float *, double *, Ctl *, int);
 template __global__ void k_chain_schur<double>(DevSym, double *, Ctl *, int);
 template __global__ void k_chain_schur<float>(DevSym, float *, Ctl *, int);
-template __global__ void k_chain_invert<double>(DevSym, double *, Ctl *, int);
-template __global__ void k_chain_invert<float>(DevSym, float *, Ctl *, int);
+template __global__ void k_chain_invert<double, 1, 1>(DevSym, double *, Ctl *, int);
+template __global__ void k_chain_invert<double, 2, 2>(DevSym, double *, Ctl *, int);
+template __global__ void k_chain_invert<double, 3, 3>(DevSym, double *, Ctl *, int);
+template __global__ void k_chain_invert<double, 4, 3>(DevSym, double *, Ctl *, int);
+template __global__ void k_chain_invert<float, 1, 1>(DevSym, float *, Ctl *, int);
+template __global__ void k_chain_invert<float, 2, 2>(DevSym, float *, Ctl *, int);
+template __global__ void k_chain_invert<float, 3, 3>(DevSym, float *, Ctl *, int);
+template __global__ void k_chain_invert<float, 4, 4>(DevSym, float *, Ctl *, int);
 template __global__ void k_factor_tail<double>(DevSym, double *, Ctl *, int, int, int);
 template __global__ void k_factor_tail<float>(DevSym, float *, Ctl *, int, int, int);
 template __global__ void k_tail_factor_ext<double>(DevSym, DevFlat, double *, Ctl *, int, int);

@@ -70,6 +70,9 @@ constexpr bool chain_tiles_fit() {
                                      ((m + ChainTiles<T>::tc - 1) / ChainTiles<T>::tc) <= ChainTiles<T>::threads;
 }
 static_assert(chain_tiles_fit<float>() && chain_tiles_fit<double>(), "dense chain does not fit the registers");
+// the smallest square tile (at most 3 x 3 blocks) whose 1024 cover a chain of
+// m nodes, 4: the largest tile, for longer chains
+inline int chain_tile(int m) { return m <= 32 ? 1 : m <= 64 ? 2 : m <= 96 ? 3 : 4; }
 // lanes per destination block in the cooperative narrow-level factorisation
 constexpr int kCoopLanes = 4;
 // most chunks of update pairs on one tail level of the single-network solver

@@ -19,7 +19,7 @@ template <typename T> __global__ void k_factor_tail_flat(DevSym Y, DevFlat F, T 
 template <typename T> __global__ void k_factor_parts_flat(DevSym Y, DevFlat F, T *blk, Ctl *ctl, int gate);
 template <typename T> __global__ void k_factor_parts(DevSym Y, T *blk, Ctl *ctl, int gate);
 template <typename T> __global__ void k_chain_schur(DevSym Y, T *blk, Ctl *ctl, int gate);
-template <typename T> __global__ void k_chain_invert(DevSym Y, T *blk, Ctl *ctl, int gate);
+template <typename T, int TR, int TC> __global__ void k_chain_invert(DevSym Y, T *blk, Ctl *ctl, int gate);
 __global__ void k_flows(DevNet N, DevState S, const FlowBranch *br, int nL, double *out);
 template <typename T> __global__ void k_fwd_parts(DevSym Y, const T *blk, double *x, Ctl *ctl, int gate);
 template <typename T> __global__ void k_fwd_parts_lds(DevSym Y, DevParts P, const T *blk, double *x, Ctl *ctl, int gate);

@@ -31,8 +31,15 @@ constexpr int kChainMax = 128;
 // LDS staging (slots are 15-bit in FlatTail::fl_s)
 constexpr int kFlatStageMax = 32767;
 constexpr int kChainMaxF64 = 101;
-// widest elimination-tree level the dense top block may take
-constexpr int kTopWidth = 1;
+// widest elimination-tree level that a dense top block of m nodes with it may
+// take.  A level outside costs a factor step and two sweep steps, a node
+// inside one more step of the inverse, whose work grows with m: on 1,888
+// buses (FP64, one network) 2,975 us at width 1 throughout, 2,705 here, 3,220
+// at width 8; on 14 buses (24 scenarios, FP64) 166, 132, 144 us.  Two nodes
+// wide up to pairs_to nodes: 64, where the inverse is 1024 threads wide; 16
+// for the batch's LDS-resident topologies, whose 256 threads then hold a
+// block each (118 buses, 333 scenarios, FP64: 18 nodes 809 us, 16 735).
+constexpr int top_width(int m, int pairs_to) { return m <= 16 ? 3 : m <= pairs_to ? 2 : 1; }
 // elimination-tree levels narrower than this run inside one workgroup (the
 // single-network solver's tail); the levels below it form subtree groups
 constexpr int kTailWidth = 64;
@@ -119,12 +126,11 @@ struct Symbolic {
     }
 };
 
-// chain_cap: most nodes of the dense top factored as one block (0: none);
-// top_width: widest elimination-tree level it may take
-Symbolic analyze(const pf_network &net, const YPattern &yp, int tail_width, int chain_cap, int top_width);
+// chain_cap: most nodes of the dense top factored as one block (0: none)
+Symbolic analyze(const pf_network &net, const YPattern &yp, int tail_width, int chain_cap, int pairs_to = 64);
 
 // chooses the dense top of an analysed network anew
-void dense_top(Symbolic &s, int chain_cap, int top_width);
+void dense_top(Symbolic &s, int chain_cap, int pairs_to);
 
 constexpr int kChunkPairs = 16;
 constexpr int kChunkDiag = 1 << 30, kChunkMask = kChunkDiag - 1;

@@ -184,8 +184,7 @@ pf_status pf_solver::build() {
     // elimination-tree level, levels narrower than kPlainTailWidth nodes in
     // one workgroup, no dense chain and no subtree groups
     const int chain_cap = opt.precision == PF_MIXED ? ChainTiles<float>::cap : ChainTiles<double>::cap;
-    sym = analyze(net, yp, opt.lu_blocked ? kTailWidth : kPlainTailWidth, opt.lu_blocked ? chain_cap : 0,
-                  kTopWidth);
+    sym = analyze(net, yp, opt.lu_blocked ? kTailWidth : kPlainTailWidth, opt.lu_blocked ? chain_cap : 0);
     if (!sym.level_ordered() || (sym.ch_m > 0 && sym.tail_start > sym.nlev_s)) {
         g_last_error = "symbolic analysis: nodes not numbered level by level, or chain outside the tail";
         return PF_INVALID_ARG;
@@ -549,7 +548,15 @@ pf_status pf_solver::enqueue_lu(T *blk, int gate) {
     if (sym.ch_m > 0) {   // the dense chain: Schur complement across the GPU, then its inverse
         const int ne = sym.fd_ptr[sym.n] - sym.fd_ptr[sym.ch_c0];
         k_chain_schur<T><<<(ne + 15) / 16, 256, 0, stream>>>(dy, blk, ctl, gate);
-        k_chain_invert<T><<<1, ChainTiles<T>::threads, 0, stream>>>(dy, blk, ctl, gate);
+        const int tile = chain_tile(sym.ch_m), tiles = (sym.ch_m + tile - 1) / tile;
+        const int threads = tile == 4 ? ChainTiles<T>::threads : (tiles * tiles + 63) / 64 * 64;
+        switch (tile) {
+            case 1: k_chain_invert<T, 1, 1><<<1, threads, 0, stream>>>(dy, blk, ctl, gate); break;
+            case 2: k_chain_invert<T, 2, 2><<<1, threads, 0, stream>>>(dy, blk, ctl, gate); break;
+            case 3: k_chain_invert<T, 3, 3><<<1, threads, 0, stream>>>(dy, blk, ctl, gate); break;
+            default:
+                k_chain_invert<T, ChainTiles<T>::tr, ChainTiles<T>::tc><<<1, threads, 0, stream>>>(dy, blk, ctl, gate);
+        }
     }
     HIPCHK(hipGetLastError());
     return PF_OK;

@@ -299,7 +299,7 @@ Symbolic analyze_order(const pf_network &net, const YPattern &yp, int tail_width
 // contiguous range of nodes (lvl_nodes is the identity) and the factor
 // program, the row structures and the flattened destinations of a level are
 // contiguous too.
-Symbolic analyze(const pf_network &net, const YPattern &yp, int tail_width, int chain_cap, int top_width) {
+Symbolic analyze(const pf_network &net, const YPattern &yp, int tail_width, int chain_cap, int pairs_to) {
     const int nB = net.nB, sl = net.slack;
     const int n = nB - 1;
     auto blk = [&](int k) { return k - (k > sl ? 1 : 0); };
@@ -320,20 +320,20 @@ Symbolic analyze(const pf_network &net, const YPattern &yp, int tail_width, int 
     std::vector<int> perm(n);
     for (int t = 0; t < n; t++) perm[t] = md[by_level[t]];
     Symbolic s = analyze_order(net, yp, tail_width, perm, gp, gi);
-    dense_top(s, chain_cap, top_width);
+    dense_top(s, chain_cap, pairs_to);
     return s;
 }
 
-void dense_top(Symbolic &s, int chain_cap, int top_width) {
+void dense_top(Symbolic &s, int chain_cap, int pairs_to) {
     const int n = s.n;
-    // dense top: the last elimination-tree levels, each at most top_width
+    // dense top: the last elimination-tree levels, each at most top_width()
     // nodes wide, at most chain_cap nodes in all.  They are factored as one
     // dense block (its Schur complement, inverted), so the level walks end
     // below them; entries of the block outside the pattern of L are zero.
     int m = 0, taken = 0;
     while (taken < s.nlev) {
         const int l = s.nlev - 1 - taken, w = s.lvl_ptr[l + 1] - s.lvl_ptr[l];
-        if (w > top_width || m + w > chain_cap) break;
+        if (w > top_width(m + w, pairs_to) || m + w > chain_cap) break;
         m += w;
         taken++;
     }

@@ -382,3 +382,27 @@ def test_dense_lu_singular(pf, cases):
     with pytest.raises(pf.PfError) as e:
         s.lu_solve(V, np.zeros(net.nB), None, np.ones(net.nB - 1 + net.nPQ))
     assert e.value.status == pf.PF_SINGULAR
+
+
+@pytest.mark.parametrize("copies,precision", [(1, "fp64"), (8, "fp64"), (8, "mixed"), (24, "mixed"), (40, "fp64"),
+                                              (128, "fp64"), (128, "mixed")])
+def test_lu_solve_dense_tops(pf, synth, tmp_path, copies, precision):
+    """The sparse factor over networks whose dense tops take each tile of the
+    register inverse: the FP64 residual of a solve, in the binding's own
+    Jacobian, to the accuracy of FP64 and of FP32 with two FP64 refinements."""
+    known = {1: synth.case118, 8: synth.case944, 128: synth.case15104}
+    path = str(tmp_path / "net.cdfx")
+    synth.write_cdf(known[copies]() if copies in known else synth.multi_copy(copies, 118000, 2 * copies, copies),
+                    path, wide=True)
+    net = pf.Network(path)
+    _say("dense top", copies, precision, pf.SymbolicProbe(net).chain)
+    s = _solver(pf, net, precision=pf.MIXED if precision == "mixed" else pf.FP64)
+    V = 1.0 + 0.01 * np.random.default_rng(1).standard_normal(net.nB)
+    th = 0.05 * np.random.default_rng(2).standard_normal(net.nB)
+    rp, cj, v = s.jacobian(V, th, None)
+    n = len(rp) - 1
+    b = np.random.default_rng(4).standard_normal(n)
+    x = s.lu_solve(V, th, None, b)
+    r = np.zeros(n)
+    np.add.at(r, np.repeat(np.arange(n), np.diff(rp)), v * x[cj])
+    assert np.abs(r - b).max() <= 1e-9 * np.abs(v).max() * np.abs(x).max()
