@@ -20,14 +20,13 @@
 #include "pf_internal.hpp"
 
 typedef __bf16 bf16;
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace pf {
 
 enum { EPI_STORE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_DGELU = 3 };
-
-constexpr int BM = 64, BN = 64, BK = 32, LDS_K = BK + 8;   // +8: rows land on different banks
 
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 __device__ __forceinline__ float gelu_grad(float z) {
@@ -36,72 +35,116 @@ __device__ __forceinline__ float gelu_grad(float z) {
     return cdf + z * pdf;
 }
 
+// Tile of TS x TS outputs, TK of the K dimension staged at a time: each
+// thread then stages two 8-element vectors of either operand.
+template <int TS> constexpr int kTileK = TS == 64 ? 64 : 128;
+
+// The two vectors of 8 that a thread stages of an operand's tile (rows r0 ..
+// of R, k0 .. of K).  KMAJOR: stored [R x K], vectors along k, one row's 16
+// bytes each; else stored [K x R], vectors along the rows for two successive
+// k, written to LDS as (k, k + 1) pairs.
+template <int TS, bool KMAJOR>
+struct TileStage {
+    static constexpr int TK = kTileK<TS>, LD = TK + 8;   // +8: rows land on different banks
+    bf16x8 v[2];
+    int at[2];
+    __device__ __forceinline__ void load(const bf16 *__restrict__ A, int ld, int r0, int R, int k0, int K, int t) {
+        const bf16x8 zero8 = {};
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            int r, k;
+            if (KMAJOR) {
+                const int q = t + 256 * u;
+                r = q / (TK / 8);
+                k = q % (TK / 8) * 8;
+            } else {
+                r = t % (TS / 8) * 8;
+                k = t / (TS / 8) * 2 + u;
+            }
+            at[u] = r * LD + k;
+            const bool in = r0 + r < R && k0 + k < K;
+            v[u] = in ? *reinterpret_cast<const bf16x8 *>(KMAJOR ? A + (size_t)(r0 + r) * ld + k0 + k
+                                                                 : A + (size_t)(k0 + k) * ld + r0 + r)
+                      : zero8;
+        }
+    }
+    __device__ __forceinline__ void store(bf16 *s) const {
+        if (KMAJOR) {
+            *reinterpret_cast<bf16x8 *>(s + at[0]) = v[0];
+            *reinterpret_cast<bf16x8 *>(s + at[1]) = v[1];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                bf16x2 p;
+                p[0] = v[0][i];
+                p[1] = v[1][i];
+                *reinterpret_cast<bf16x2 *>(s + at[0] + i * LD) = p;
+            }
+        }
+    }
+};
+
 // C[M x N] = op(A)[M x K] * op(B)[K x N], bf16 operands, fp32 accumulate.
 //   TA = false: A row-major [M x K] (lda);  TA = true: A stored [K x M].
 //   TB = false: B row-major [K x N] (ldb);  TB = true: B stored [N x K].
 // Every dimension is a multiple of 8 (checked on the host), so 16-byte
 // loads along the contiguous dimension never straddle the edge.
-// 256 threads: 4 waves, each a 32x32 quarter of the 64x64 tile as 2x2
-// MFMA 16x16x32 blocks.
-template <bool TA, bool TB, int EPI>
+// 256 threads: 4 waves, each a quarter of the tile in MFMA 16x16x32 blocks
+// (2 x 2 of them at TS = 64, one at 32).  At these sizes a workgroup waits
+// for its loads, not for the matrix cores, so the next tile's vectors are in
+// registers while this one's are multiplied, and products of few tiles take
+// the small one (gemm()).  An output's sum runs through K in the same steps of
+// 32 whatever the tile.  256 x 512 outputs, K = 2,832: 86 us with 64-wide
+// tiles of 32 and no loads ahead, 20 now.
+template <bool TA, bool TB, int EPI, int TS>
 __global__ void __launch_bounds__(256) k_gemm(int M, int N, int K, const bf16 *__restrict__ A, int lda,
                                               const bf16 *__restrict__ B, int ldb, float *__restrict__ C,
                                               int ldc, bf16 *__restrict__ Cb, int ldcb,
                                               const float *__restrict__ bias, const float *__restrict__ Zs) {
-    __shared__ __align__(16) bf16 As[BM][LDS_K];
-    __shared__ __align__(16) bf16 Bs[BN][LDS_K];
+    constexpr int TK = kTileK<TS>, LD = TK + 8, W = TS / 32;   // W x W blocks a wave
+    __shared__ __align__(16) bf16 As[TS * LD];
+    __shared__ __align__(16) bf16 Bs[TS * LD];
     const int t = threadIdx.x;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int m0 = blockIdx.y * TS, n0 = blockIdx.x * TS;
     const int w = t >> 6, l = t & 63;
-    const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-    f32x4 acc[2][2];
-    for (int i = 0; i < 2; i++)
-        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8 zero8 = {};
-    for (int k0 = 0; k0 < K; k0 += BK) {
-        // ---- stage A tile as As[m][k]
-        if (!TA) {
-            const int m = t >> 2, kk = (t & 3) * 8;
-            bf16x8 v = zero8;
-            if (m0 + m < M && k0 + kk < K) v = *reinterpret_cast<const bf16x8 *>(A + (size_t)(m0 + m) * lda + k0 + kk);
-            *reinterpret_cast<bf16x8 *>(&As[m][kk]) = v;
-        } else {
-            const int kk = t >> 3, mm = (t & 7) * 8;
-            bf16x8 v = zero8;
-            if (k0 + kk < K && m0 + mm < M) v = *reinterpret_cast<const bf16x8 *>(A + (size_t)(k0 + kk) * lda + m0 + mm);
-#pragma unroll
-            for (int i = 0; i < 8; i++) As[mm + i][kk] = v[i];
-        }
-        // ---- stage B tile as Bs[n][k]
-        if (TB) {
-            const int n = t >> 2, kk = (t & 3) * 8;
-            bf16x8 v = zero8;
-            if (n0 + n < N && k0 + kk < K) v = *reinterpret_cast<const bf16x8 *>(B + (size_t)(n0 + n) * ldb + k0 + kk);
-            *reinterpret_cast<bf16x8 *>(&Bs[n][kk]) = v;
-        } else {
-            const int kk = t >> 3, nn = (t & 7) * 8;
-            bf16x8 v = zero8;
-            if (k0 + kk < K && n0 + nn < N) v = *reinterpret_cast<const bf16x8 *>(B + (size_t)(k0 + kk) * ldb + n0 + nn);
-#pragma unroll
-            for (int i = 0; i < 8; i++) Bs[nn + i][kk] = v[i];
-        }
+    const int wm = (w >> 1) * (TS / 2), wn = (w & 1) * (TS / 2);
+    f32x4 acc[W][W];
+    for (int i = 0; i < W; i++)
+        for (int j = 0; j < W; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    TileStage<TS, !TA> sa;
+    TileStage<TS, TB> sb;
+    sa.load(A, lda, m0, M, 0, K, t);
+    sb.load(B, ldb, n0, N, 0, K, t);
+    for (int k0 = 0; k0 < K; k0 += TK) {
+        sa.store(As);
+        sb.store(Bs);
         __syncthreads();
-        bf16x8 a[2], b[2];
+        if (k0 + TK < K) {
+            sa.load(A, lda, m0, M, k0 + TK, K, t);
+            sb.load(B, ldb, n0, N, k0 + TK, K, t);
+        }
 #pragma unroll
-        for (int i = 0; i < 2; i++) a[i] = *reinterpret_cast<const bf16x8 *>(&As[wm + 16 * i + (l & 15)][8 * (l >> 4)]);
+        for (int kk = 0; kk < TK; kk += 32) {
+            bf16x8 a[W], b[W];
 #pragma unroll
-        for (int j = 0; j < 2; j++) b[j] = *reinterpret_cast<const bf16x8 *>(&Bs[wn + 16 * j + (l & 15)][8 * (l >> 4)]);
+            for (int i = 0; i < W; i++)
+                a[i] = *reinterpret_cast<const bf16x8 *>(&As[(wm + 16 * i + (l & 15)) * LD + kk + 8 * (l >> 4)]);
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+            for (int j = 0; j < W; j++)
+                b[j] = *reinterpret_cast<const bf16x8 *>(&Bs[(wn + 16 * j + (l & 15)) * LD + kk + 8 * (l >> 4)]);
 #pragma unroll
-            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < W; i++)
+#pragma unroll
+                for (int j = 0; j < W; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
         __syncthreads();
     }
     // ---- epilogue: lane l owns rows 4*(l/16)+v, column l%16 of each 16x16 block
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < W; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < W; j++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = m0 + wm + 16 * i + 4 * (l >> 4) + v;
@@ -125,22 +168,25 @@ __global__ void __launch_bounds__(256) k_gemm(int M, int N, int K, const bf16 *_
             }
 }
 
-__global__ void k_norm_in(const float *X, int B, int n, const float *mean, const float *inv_std, bf16 *Xn) {
+// rows idx[0 .. B) of X (idx null: rows 0 .. B), normalised
+__global__ void k_norm_in(const float *X, const int *idx, int B, int n, const float *mean, const float *inv_std,
+                          bf16 *Xn) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)B * n) return;
-    const int c = (int)(i % n);
-    Xn[i] = (bf16)((X[i] - mean[c]) * inv_std[c]);
+    const int r = (int)(i / n), c = (int)(i - (size_t)r * n);
+    Xn[i] = (bf16)((X[(size_t)(idx ? idx[r] : r) * n + c] - mean[c]) * inv_std[c]);
 }
 
-// dY = 2 (Y - (T - mean)/std) / (B n); loss partial sums per block
-__global__ void k_out_grad(const float *Y, const float *T, int B, int n, const float *mean, const float *inv_std,
-                           float *dY, bf16 *dYb, float *loss_part) {
+// dY = 2 (Y - (T - mean)/std) / (B n), T's rows by idx as above; loss partial
+// sums per block
+__global__ void k_out_grad(const float *Y, const float *T, const int *idx, int B, int n, const float *mean,
+                           const float *inv_std, float *dY, bf16 *dYb, float *loss_part) {
     __shared__ float red[256];
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     float e2 = 0.f;
     if (i < (size_t)B * n) {
-        const int c = (int)(i % n);
-        const float d = Y[i] - (T[i] - mean[c]) * inv_std[c];
+        const int r = (int)(i / n), c = (int)(i - (size_t)r * n);
+        const float d = Y[i] - (T[(size_t)(idx ? idx[r] : r) * n + c] - mean[c]) * inv_std[c];
         const float g = 2.f * d / ((float)B * (float)n);
         dY[i] = g;
         dYb[i] = (bf16)g;
@@ -155,16 +201,30 @@ __global__ void k_out_grad(const float *Y, const float *T, int B, int n, const f
     if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0];
 }
 
-// column sums (bias gradient): db[c] = sum_r dZ[r, c]
-__global__ void k_colsum(const float *dZ, int B, int n, float *db) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
+// column sums (bias gradient): db[c] = sum_r dZ[r, c], in row order (AdamW
+// divides small gradients by their own size, so another order of the same
+// sum shows in the weights).  A wave per 64 columns, a thread each, 64 rows in
+// flight: the loads' latency, 60 us for 256 x 512 with a few in flight, is
+// paid once per 64 rows, 4.6 us.
+__global__ void __launch_bounds__(64) k_colsum(const float *dZ, int B, int n, float *db) {
+    constexpr int U = 64;
+    const int c = (int)blockIdx.x * 64 + (int)threadIdx.x;
     if (c >= n) return;
     float s = 0.f;
-    for (int r = 0; r < B; r++) s += dZ[(size_t)r * n + c];
+    int r = 0;
+    for (; r + U <= B; r += U) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = (dZ + (size_t)(r + u) * n)[c];
+#pragma unroll
+        for (int u = 0; u < U; u++) s += v[u];
+    }
+    for (; r < B; r++) s += dZ[(size_t)r * n + c];
     db[c] = s;
 }
 
-__global__ void k_adamw(float *p, const float *g, float *m, float *v, size_t n, float lr, float b1, float b2,
+// one AdamW update, and the bf16 copy of the parameters that the products read
+__global__ void k_adamw(float *p, bf16 *pb, const float *g, float *m, float *v, size_t n, float lr, float b1, float b2,
                         float eps, float wd, float bc1, float bc2) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -174,19 +234,14 @@ __global__ void k_adamw(float *p, const float *g, float *m, float *v, size_t n, 
     m[i] = mi;
     v[i] = vi;
     const float mh = mi / bc1, vh = vi / bc2;
-    p[i] -= lr * (mh / (sqrtf(vh) + eps) + wd * p[i]);
+    const float pi = p[i] - lr * (mh / (sqrtf(vh) + eps) + wd * p[i]);
+    p[i] = pi;
+    pb[i] = (bf16)pi;
 }
 
 __global__ void k_to_bf16(const float *src, bf16 *dst, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = (bf16)src[i];
-}
-
-__global__ void k_gather_rows(const float *src, const int *idx, int B, int n, float *dst) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)B * n) return;
-    const size_t r = i / n, c = i % n;
-    dst[i] = src[(size_t)idx[r] * n + c];
 }
 
 __global__ void k_denorm(const float *Y, int B, int n, const float *mean, const float *std, float *out) {
@@ -238,7 +293,12 @@ struct pf_warmstart {
     hipStream_t stream = nullptr;
     std::vector<void *> allocs, ws_allocs;
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
-    std::vector<bf16 *> Wb;
+    bf16 *pb = nullptr;        // the parameters in bf16, laid out as p
+    std::vector<bf16 *> Wb;    // its layers' weights
+    float *fX = nullptr, *fT = nullptr;   // fit's resident rows and permutation, kept up to kFitKeep bytes
+    int *fperm = nullptr;
+    size_t fit_cap = 0;        // floats at fX (then fT)
+    int perm_cap = 0;
     float *xm = nullptr, *xis = nullptr, *ym = nullptr, *yis = nullptr, *ys = nullptr;
     // workspace
     float *X = nullptr, *T = nullptr, *Yp = nullptr, *Yo = nullptr, *loss_part = nullptr;
@@ -259,6 +319,8 @@ struct pf_warmstart {
     ~pf_warmstart() {
         for (void *q : ws_allocs) (void)hipFree(q);
         for (void *q : allocs) (void)hipFree(q);
+        (void)hipFree(fX);
+        (void)hipFree(fperm);
         if (stream) (void)hipStreamDestroy(stream);
     }
     pf_status ensure(int B);
@@ -266,8 +328,9 @@ struct pf_warmstart {
     template <bool TA, bool TB, int EPI>
     pf_status gemm(int M_, int N_, int K_, const bf16 *A, int lda, const bf16 *B, int ldb, float *C, int ldc,
                    bf16 *Cb, int ldcb, const float *bias, const float *Zs);
-    pf_status forward(int B);
-    pf_status backward(int B, double *loss);
+    pf_status forward(int B, const float *rows, const int *idx);
+    pf_status backward(int B, const float *targets, const int *idx, float *parts, double *loss);
+    pf_status fit_room(int n);
 };
 
 pf_status pf_warmstart::ensure(int B) {
@@ -297,11 +360,31 @@ pf_status pf_warmstart::ensure(int B) {
     return PF_OK;
 }
 
-pf_status pf_warmstart::sync_bf16() {
-    for (int l = 0; l < n_layers; l++) {
-        size_t n = (size_t)K[l] * N[l];
-        k_to_bf16<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(p + w_off[l], Wb[l], n);
+// Room for n rows of features and targets on the device: a small data set's
+// stays with the network from one fit to the next.
+constexpr size_t kFitKeep = 256u << 20;
+pf_status pf_warmstart::fit_room(int n) {
+    const size_t nx = (size_t)n * n_in, need = nx + (size_t)n * n_out;
+    if (need > fit_cap) {
+        MHIP(hipFree(fX));
+        fX = nullptr;
+        fit_cap = 0;
+        MHIP(hipMalloc((void **)&fX, sizeof(float) * need));
+        fit_cap = need;
     }
+    fT = fX + nx;
+    if (n > perm_cap) {
+        MHIP(hipFree(fperm));
+        fperm = nullptr;
+        perm_cap = 0;
+        MHIP(hipMalloc((void **)&fperm, sizeof(int) * n));
+        perm_cap = n;
+    }
+    return PF_OK;
+}
+
+pf_status pf_warmstart::sync_bf16() {
+    k_to_bf16<<<(unsigned)((n_params + 255) / 256), 256, 0, stream>>>(p, pb, n_params);
     MHIP(hipGetLastError());
     return PF_OK;
 }
@@ -310,15 +393,23 @@ template <bool TA, bool TB, int EPI>
 pf_status pf_warmstart::gemm(int M_, int N_, int K_, const bf16 *A, int lda, const bf16 *B, int ldb, float *C,
                              int ldc, bf16 *Cb, int ldcb, const float *bias, const float *Zs) {
     if (M_ % 8 || N_ % 8 || K_ % 8) return PF_INVALID_ARG;
-    dim3 grid((N_ + BN - 1) / BN, (M_ + BM - 1) / BM);
-    k_gemm<TA, TB, EPI><<<grid, 256, 0, stream>>>(M_, N_, K_, A, lda, B, ldb, C, ldc, Cb, ldcb, bias, Zs);
+    // 64-wide tiles where they give every CU one; else four times as many of 32
+    // (256 x 1,888 outputs, K = 512, in 120 tiles of 64: 18 us; in 472 of 32: 7)
+    const int wide = ((N_ + 63) / 64) * ((M_ + 63) / 64);
+    if (wide >= 256) {
+        dim3 grid((N_ + 63) / 64, (M_ + 63) / 64);
+        k_gemm<TA, TB, EPI, 64><<<grid, 256, 0, stream>>>(M_, N_, K_, A, lda, B, ldb, C, ldc, Cb, ldcb, bias, Zs);
+    } else {
+        dim3 grid((N_ + 31) / 32, (M_ + 31) / 32);
+        k_gemm<TA, TB, EPI, 32><<<grid, 256, 0, stream>>>(M_, N_, K_, A, lda, B, ldb, C, ldc, Cb, ldcb, bias, Zs);
+    }
     MHIP(hipGetLastError());
     return PF_OK;
 }
 
-pf_status pf_warmstart::forward(int B) {
+pf_status pf_warmstart::forward(int B, const float *rows, const int *idx) {
     size_t nx = (size_t)B * n_in;
-    k_norm_in<<<(unsigned)((nx + 255) / 256), 256, 0, stream>>>(X, B, n_in, xm, xis, Xn);
+    k_norm_in<<<(unsigned)((nx + 255) / 256), 256, 0, stream>>>(rows, idx, B, n_in, xm, xis, Xn);
     MHIP(hipGetLastError());
     const bf16 *in = Xn;
     for (int l = 0; l < n_layers; l++) {
@@ -335,18 +426,19 @@ pf_status pf_warmstart::forward(int B) {
     return PF_OK;
 }
 
-pf_status pf_warmstart::backward(int B, double *loss) {
+// loss partial sums go to parts; *loss (may be null) waits for them
+pf_status pf_warmstart::backward(int B, const float *targets, const int *idx, float *parts_d, double *loss) {
     size_t ny = (size_t)B * n_out;
     unsigned nb = (unsigned)((ny + 255) / 256);
     int cur = 0;
-    k_out_grad<<<nb, 256, 0, stream>>>(Yp, T, B, n_out, ym, yis, dZf[cur], dZb[cur], loss_part);
+    k_out_grad<<<nb, 256, 0, stream>>>(Yp, targets, idx, B, n_out, ym, yis, dZf[cur], dZb[cur], parts_d);
     MHIP(hipGetLastError());
     for (int l = n_layers - 1; l >= 0; l--) {
         const bf16 *hin = (l == 0) ? Xn : H[l - 1];
         // dW_l = H_{l-1}^T dZ_l : [K_l x N_l], reduction over the batch
         MCHK((gemm<true, false, EPI_STORE>(K[l], N[l], B, hin, K[l], dZb[cur], N[l], g + w_off[l], N[l], nullptr,
                                            0, nullptr, nullptr)));
-        k_colsum<<<(N[l] + 255) / 256, 256, 0, stream>>>(dZf[cur], B, N[l], g + b_off[l]);
+        k_colsum<<<(N[l] + 63) / 64, 64, 0, stream>>>(dZf[cur], B, N[l], g + b_off[l]);
         MHIP(hipGetLastError());
         if (l > 0) {
             // dZ_{l-1} = (dZ_l W_l^T) * gelu'(Z_{l-1})
@@ -357,7 +449,7 @@ pf_status pf_warmstart::backward(int B, double *loss) {
     }
     if (loss) {
         std::vector<float> parts(nb);
-        MHIP(hipMemcpyAsync(parts.data(), loss_part, sizeof(float) * nb, hipMemcpyDeviceToHost, stream));
+        MHIP(hipMemcpyAsync(parts.data(), parts_d, sizeof(float) * nb, hipMemcpyDeviceToHost, stream));
         MHIP(hipStreamSynchronize(stream));
         double s = 0;
         for (float x : parts) s += x;
@@ -410,12 +502,13 @@ pf_status pf_warmstart_create(int n_in, int n_out, int hidden, int n_hidden_laye
     MCHK(w->alloc(&w->g, off, w->allocs));
     MCHK(w->alloc(&w->m, off, w->allocs));
     MCHK(w->alloc(&w->v, off, w->allocs));
+    MCHK(w->alloc(&w->pb, off, w->allocs));
     MHIP(hipMemcpy(w->p, h.data(), sizeof(float) * off, hipMemcpyHostToDevice));
     MHIP(hipMemset(w->m, 0, sizeof(float) * off));
     MHIP(hipMemset(w->v, 0, sizeof(float) * off));
     MHIP(hipMemset(w->g, 0, sizeof(float) * off));
     w->Wb.resize(w->n_layers);
-    for (int l = 0; l < w->n_layers; l++) MCHK(w->alloc(&w->Wb[l], (size_t)w->K[l] * w->N[l], w->allocs));
+    for (int l = 0; l < w->n_layers; l++) w->Wb[l] = w->pb + w->w_off[l];   // 16-byte rows: every size is a multiple of 8
     MCHK(w->alloc(&w->xm, n_in, w->allocs));
     MCHK(w->alloc(&w->xis, n_in, w->allocs));
     MCHK(w->alloc(&w->ym, n_out, w->allocs));
@@ -489,8 +582,8 @@ pf_status pf_warmstart_grad(pf_warmstart *w, const float *X, const float *Y, int
     MCHK(w->ensure(B));
     MHIP(hipMemcpyAsync(w->X, X, sizeof(float) * (size_t)B * w->n_in, hipMemcpyHostToDevice, w->stream));
     MHIP(hipMemcpyAsync(w->T, Y, sizeof(float) * (size_t)B * w->n_out, hipMemcpyHostToDevice, w->stream));
-    MCHK(w->forward(B));
-    MCHK(w->backward(B, loss));
+    MCHK(w->forward(B, w->X, nullptr));
+    MCHK(w->backward(B, w->T, nullptr, w->loss_part, loss));
     if (grads) MHIP(hipMemcpyAsync(grads, w->g, sizeof(float) * w->n_params, hipMemcpyDeviceToHost, w->stream));
     MHIP(hipStreamSynchronize(w->stream));
     return PF_OK;
@@ -505,51 +598,70 @@ pf_status pf_warmstart_fit(pf_warmstart *w, const float *X, const float *Y, int 
     w->staged = 0;   // the minibatches replace the staged rows
     MHIP(hipSetDevice(w->device));
     MCHK(w->ensure(B));
-    float *dX = nullptr, *dY = nullptr;
-    int *dperm = nullptr;
+    MCHK(w->fit_room(n));
+    float *dX = w->fX, *dY = w->fT;
+    int *dperm = w->fperm;
+    // every step's loss sums, read once an epoch
+    const int nbat = n / B;
+    const size_t nb = ((size_t)B * w->n_out + 255) / 256;
     std::vector<void *> tmp;
-    MCHK(w->alloc(&dX, (size_t)n * w->n_in, tmp));
-    MCHK(w->alloc(&dY, (size_t)n * w->n_out, tmp));
-    MCHK(w->alloc(&dperm, (size_t)n, tmp));
+    float *parts = nullptr;
+    std::vector<float> hp;
+    if (epoch_loss) {
+        MCHK(w->alloc(&parts, nb * nbat, tmp));
+        hp.resize(nb * nbat);
+    }
     pf_status st = PF_OK;
-    MHIP(hipMemcpy(dX, X, sizeof(float) * (size_t)n * w->n_in, hipMemcpyHostToDevice));
-    MHIP(hipMemcpy(dY, Y, sizeof(float) * (size_t)n * w->n_out, hipMemcpyHostToDevice));
+    auto ok = [&](hipError_t e) {
+        if (e != hipSuccess && st == PF_OK) {
+            pf::set_last_error(std::string("pf_warmstart_fit: ") + hipGetErrorString(e));
+            st = PF_DEVICE_ERROR;
+        }
+    };
+    ok(hipMemcpy(dX, X, sizeof(float) * (size_t)n * w->n_in, hipMemcpyHostToDevice));
+    ok(hipMemcpy(dY, Y, sizeof(float) * (size_t)n * w->n_out, hipMemcpyHostToDevice));
     std::vector<int> perm(n);
     for (int i = 0; i < n; i++) perm[i] = i;
     unsigned long long s = seed;
-    const int nbat = n / B;
     for (int ep = 0; ep < epochs && st == PF_OK; ep++) {
         for (int i = n - 1; i > 0; i--) {
             int j = (int)(sm64(s) % (unsigned long long)(i + 1));
             std::swap(perm[i], perm[j]);
         }
-        if (hipMemcpyAsync(dperm, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice, w->stream) != hipSuccess ||
-            hipStreamSynchronize(w->stream) != hipSuccess) {
-            st = PF_DEVICE_ERROR;
-            break;
-        }
-        double acc = 0;
+        ok(hipMemcpyAsync(dperm, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice, w->stream));
+        ok(hipStreamSynchronize(w->stream));   // perm is shuffled again for the next epoch
         for (int bi = 0; bi < nbat && st == PF_OK; bi++) {
-            const size_t nx = (size_t)B * w->n_in, ny = (size_t)B * w->n_out;
-            k_gather_rows<<<(unsigned)((nx + 255) / 256), 256, 0, w->stream>>>(dX, dperm + (size_t)bi * B, B, w->n_in, w->X);
-            k_gather_rows<<<(unsigned)((ny + 255) / 256), 256, 0, w->stream>>>(dY, dperm + (size_t)bi * B, B, w->n_out, w->T);
-            double loss = 0;
-            st = w->forward(B);
-            if (st == PF_OK) st = w->backward(B, epoch_loss ? &loss : nullptr);
+            const int *idx = dperm + (size_t)bi * B;
+            st = w->forward(B, dX, idx);
+            if (st == PF_OK) st = w->backward(B, dY, idx, parts ? parts + nb * bi : w->loss_part, nullptr);
             if (st != PF_OK) break;
             w->step++;
             const float b1 = 0.9f, b2 = 0.999f;
             const float bc1 = 1.0f - std::pow(b1, (float)w->step), bc2 = 1.0f - std::pow(b2, (float)w->step);
-            k_adamw<<<(unsigned)((w->n_params + 255) / 256), 256, 0, w->stream>>>(w->p, w->g, w->m, w->v, w->n_params,
-                                                                                 lr, b1, b2, 1e-8f, weight_decay,
-                                                                                 bc1, bc2);
-            st = w->sync_bf16();
-            acc += loss;
+            k_adamw<<<(unsigned)((w->n_params + 255) / 256), 256, 0, w->stream>>>(w->p, w->pb, w->g, w->m, w->v,
+                                                                                 w->n_params, lr, b1, b2, 1e-8f,
+                                                                                 weight_decay, bc1, bc2);
+            ok(hipGetLastError());
         }
-        if (epoch_loss) epoch_loss[ep] = acc / nbat;
+        if (epoch_loss && st == PF_OK) {
+            ok(hipMemcpyAsync(hp.data(), parts, sizeof(float) * hp.size(), hipMemcpyDeviceToHost, w->stream));
+            ok(hipStreamSynchronize(w->stream));
+            double acc = 0;
+            for (int bi = 0; bi < nbat; bi++) {
+                double l = 0;
+                for (size_t i = 0; i < nb; i++) l += hp[nb * bi + i];
+                acc += l / ((double)B * w->n_out);
+            }
+            epoch_loss[ep] = acc / nbat;
+        }
     }
-    (void)hipStreamSynchronize(w->stream);
+    ok(hipStreamSynchronize(w->stream));
     for (void *q : tmp) (void)hipFree(q);
+    if (w->fit_cap * sizeof(float) > kFitKeep) {   // a large data set's room goes back
+        (void)hipFree(w->fX);
+        w->fX = w->fT = nullptr;
+        w->fit_cap = 0;
+    }
     return st;
 }
 
@@ -560,7 +672,7 @@ pf_status pf_warmstart_predict(pf_warmstart *w, const float *X, int B, float *Y)
     MHIP(hipSetDevice(w->device));
     MCHK(w->ensure(B));
     MHIP(hipMemcpyAsync(w->X, X, sizeof(float) * (size_t)B * w->n_in, hipMemcpyHostToDevice, w->stream));
-    MCHK(w->forward(B));
+    MCHK(w->forward(B, w->X, nullptr));
     size_t ny = (size_t)B * w->n_out;
     k_denorm<<<(unsigned)((ny + 255) / 256), 256, 0, w->stream>>>(w->Yp, B, w->n_out, w->ym, w->ys, w->Yo);
     MHIP(hipGetLastError());
@@ -582,7 +694,7 @@ pf_status pf_warmstart_stage(pf_warmstart *w, const float *X, int B) {
 pf_status pf_warmstart_predict_into(pf_warmstart *w, pf_batch *b, int v_col, int th_col) {
     if (!w || !b || w->staged <= 0) return PF_INVALID_ARG;
     MHIP(hipSetDevice(w->device));
-    MCHK(w->forward(w->staged));
+    MCHK(w->forward(w->staged, w->X, nullptr));
     return batch_start_from_rows(b, w->device, w->staged, w->Yp, w->n_out, v_col, th_col, w->ym, w->ys,
                                  (void *)w->stream);
 }

@@ -176,3 +176,44 @@ def test_warm_start_predict_into_batch(pf, synth):
     w.stage(Xt)
     with pytest.raises(pf.PfError):
         w.predict_into(dev, 0, n_out8 - net.nB + 1)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("shape", [(8, 8, 8), (40, 24, 136), (264, 520, 120), (1032, 1048, 72), (1088, 1024, 64)])
+def test_gemm_bf16_tiles(pf, ta, tb, shape):
+    """Both tile widths (64 from 256 tiles of it on), at edges of their rows,
+    columns and K steps: FP32 accumulation of exact bf16 products, so within K
+    rounding units of the sum of magnitudes."""
+    import mlp_oracle as M
+    m, n, k = shape
+    _say("gemm", shape, ta, tb)
+    w = pf.WarmStart(16, 16, 16, 1)
+    rng = np.random.default_rng(3)
+    A = rng.standard_normal((k, m) if ta else (m, k)).astype(np.float32)
+    B = rng.standard_normal((n, k) if tb else (k, n)).astype(np.float32)
+    C = w.gemm_probe(A, B, ta, tb)
+    Aq, Bq = (x.astype(np.float64) for x in (M.bf16(A), M.bf16(B)))
+    Aq, Bq = (Aq.T if ta else Aq), (Bq.T if tb else Bq)
+    assert np.all(np.abs(C - Aq @ Bq) <= k * 2.0 ** -24 * (np.abs(Aq) @ np.abs(Bq)) + 1e-30)
+
+
+def test_fit_grows_and_keeps_its_rows(pf):
+    """Training calls of different sizes on one network: each starts from the
+    state the one before left, whatever room for rows is kept between them."""
+    rng = np.random.default_rng(6)
+    X = rng.standard_normal((200, 16)).astype(np.float32)
+    Y = rng.standard_normal((200, 8)).astype(np.float32)
+    out = []
+    for first in (16, 200):
+        w = pf.WarmStart(16, 8, 24, 1, seed=3)
+        if first == 200:
+            p = w.params()
+            w.fit(X, Y, epochs=1, batch=40)      # room for 200 rows before the small call
+            w2 = pf.WarmStart(16, 8, 24, 1, seed=3)
+            assert np.array_equal(p, w2.params())
+            w = w2
+        w.fit(X[:16], Y[:16], epochs=2, batch=8)
+        w.fit(X, Y, epochs=1, batch=40)
+        w.fit(X[:64], Y[:64], epochs=1, batch=8)
+        out.append(w.params())
+    assert np.array_equal(out[0], out[1]) and np.all(np.isfinite(out[0]))
