@@ -805,27 +805,35 @@ __device__ __forceinline__ void wg_set_E(const DevNet &N, Work<T> &w) {
     }
 }
 
-// One NR solve of one scenario by the whole workgroup.  Returns (via shared
-// result) iterations, converged flag and final max mismatch.
+// Starting state of one scenario
 template <typename T>
-__device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Work<T> &w, const double *Pliq,
-                      const double *Qliq, const double *Qload, const double *V0, const double *th0,
-                      int *s_it, int *s_conv, double *s_maxg, int *s_fl, B4<T> *s_chain, B4<T> *s_ck) {
+__device__ __forceinline__ void wg_start(const BatchTopo &tp, Work<T> &w, const double *Qliq, const double *V0,
+                                         const double *th0) {
     const DevNet &N = tp.N;
-    const DevSym &Y = tp.Y;
-    __shared__ unsigned long long s_maxG_bits, s_maxDx_bits;
-    __shared__ int s_bad, s_flips, s_sing;
-    const int tid = threadIdx.x;
     // a warm start sets |V| of the PQ buses and the angles of the non-slack
     // buses; PV buses start at their setpoint and the slack at its data
-    for (int k = tid; k < N.nB; k += blockDim.x) {
+    for (int k = threadIdx.x; k < N.nB; k += blockDim.x) {
         const bool pq = N.pv_of_bus[k] < 0 && k != N.slack;
         w.V[k] = pq ? V0[k] : tp.V0flat[k];
         w.th[k] = (k == N.slack) ? tp.th0flat[k] : th0[k];
         w.ql[k] = Qliq[k];
         w.isq[k] = pq ? 1 : 0;                                   // initLim: PQ buses only
     }
-    for (int i = tid; i < N.nPV; i += blockDim.x) w.limQ[i] = 0;
+    for (int i = threadIdx.x; i < N.nPV; i += blockDim.x) w.limQ[i] = 0;
+}
+
+// One NR solve of one scenario by the whole workgroup from the state in w.
+// Returns (via shared result) iterations, converged flag, final max mismatch,
+// flips and whether a pivot failed (s_end, may be null).
+template <typename T>
+__device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Work<T> &w, const double *Pliq,
+                      const double *Qliq, const double *Qload,
+                      int *s_it, int *s_conv, double *s_maxg, int *s_fl, int *s_end, B4<T> *s_chain, B4<T> *s_ck) {
+    const DevNet &N = tp.N;
+    const DevSym &Y = tp.Y;
+    __shared__ unsigned long long s_maxG_bits, s_maxDx_bits;
+    __shared__ int s_bad, s_flips, s_sing;
+    const int tid = threadIdx.x;
     if (tid == 0) {
         s_maxDx_bits = 0;
         s_flips = 0;
@@ -889,7 +897,7 @@ __device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Wo
             conv = 1;
             break;
         }
-        if (!(maxG < J.diverge)) break;                   // NaN or diverging: give up this start
+        if (J.diverge > 0 && !(maxG < J.diverge)) break;  // NaN or diverging: give up this start
         // Jacobian blocks, four slots a thread at a time so that their index
         // loads are in flight together
         constexpr int JF = 4;
@@ -1018,6 +1026,7 @@ __device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Wo
         *s_conv = conv;
         *s_maxg = maxG;
         *s_fl = s_flips;
+        if (s_end) *s_end = s_sing;
     }
     __syncthreads();
 }
@@ -1088,8 +1097,8 @@ __global__ void __launch_bounds__(MAXT, (batch_min_waves<T, MODE, MAXT>())) k_ba
         // when it does not converge, the flat-start fallback
         for (int attempt = warm ? 0 : 1; attempt < 2; ++attempt) {
             const bool from_warm = attempt == 0;
-            wg_nr(tp, J, w, Pl, Ql, Qd, from_warm ? J.V0 + off : tp.V0flat,
-                  from_warm ? J.th0 + off : tp.th0flat, &s_it, &s_conv, &s_maxg, &s_fl, s_chain,
+            wg_start(tp, w, Ql, from_warm ? J.V0 + off : tp.V0flat, from_warm ? J.th0 + off : tp.th0flat);
+            wg_nr(tp, J, w, Pl, Ql, Qd, &s_it, &s_conv, &s_maxg, &s_fl, (int *)nullptr, s_chain,
                   MODE == 2 ? nullptr : s_ck);
             total_it += s_it;
             if (s_conv) break;                              // shared: uniform over the workgroup
@@ -1110,6 +1119,48 @@ __global__ void __launch_bounds__(MAXT, (batch_min_waves<T, MODE, MAXT>())) k_ba
     }
 }
 
+// The whole NR loop of the single-network solver in one workgroup, the
+// working set in LDS: from the solver's state and back to it, the outcome
+// into *out (host memory).  A pass across the GPU is some twenty dependent
+// launches, about 100 us whatever the size; here it is a barrier a step, 22 us
+// at 14 buses and 50 at 118 (FP64), bound by the chain of levels.  A solve
+// with its state read, FP64, 4 passes at 14 buses and 6 above, replayed graphs
+// across the GPU -> one workgroup: 14 buses 431 -> 170 us, 57 buses
+// 488 -> 212, 118 buses 704 -> 384, 236 buses 904 -> 635; mixed 354 buses
+// 1,252 -> 949, the largest that fits.  The line is the LDS: all that fits is
+// faster here.
+template <typename T>
+__global__ void __launch_bounds__(512) k_solve_wg(BatchTopo tp, BatchJob J, DevState S, Ctl *out) {
+    extern __shared__ __align__(16) char smem[];
+    __shared__ int s_it, s_conv, s_fl, s_end;
+    __shared__ B4<T> s_chain[4 * kBatchChain + 2];
+    __shared__ double s_maxg;
+    const DevNet &N = tp.N;
+    Work<T> w = carve<T>(smem, N.nB, tp.Y.n, N.nPV, tp.nblk);
+    for (int k = threadIdx.x; k < N.nB; k += blockDim.x) {
+        w.V[k] = S.V[k];
+        w.th[k] = S.th[k];
+        w.ql[k] = S.QliqLim[k];
+        w.isq[k] = S.isq[k];
+    }
+    for (int i = threadIdx.x; i < N.nPV; i += blockDim.x) w.limQ[i] = S.limQ[i];
+    wg_nr(tp, J, w, S.Pliq, S.Qliq, S.Qload, &s_it, &s_conv, &s_maxg, &s_fl, &s_end, s_chain, (B4<T> *)nullptr);
+    for (int k = threadIdx.x; k < N.nB; k += blockDim.x) {
+        S.V[k] = w.V[k];
+        S.th[k] = w.th[k];
+        S.E[k] = w.E[k];
+        S.QliqLim[k] = w.ql[k];
+        S.isq[k] = w.isq[k];
+    }
+    for (int i = threadIdx.x; i < N.nPV; i += blockDim.x) S.limQ[i] = w.limQ[i];
+    if (threadIdx.x == 0) {
+        out->it = s_it + s_end;   // a pass whose factors fail counts, its step is not taken
+        out->done = s_conv;
+        out->singular = s_end;
+        out->maxG = s_maxg;
+        out->flips = s_fl;
+    }
+}
 
 // ------------------------------------------------------------ fixed scratch
 // The allocation-free batch entry point keeps its per-call tables (packed
@@ -1250,6 +1301,39 @@ namespace {
 // (80 KiB) 1,740 us in LDS, 1,140 us in MODE 1.
 constexpr long long kLdsLimit = 75 * 1024;
 }  // namespace
+
+// LDS bytes of k_solve_wg for a network, 0 where it does not run (the working
+// set beyond the device's LDS, or a dense top past its staging)
+long long pf::solve_wg_lds(const pf_network &net, const Symbolic &s, bool mixed, long long max_lds) {
+    const long long b = mixed ? work_bytes<float>(net.nB, s.n, net.nPV, s.nblk())
+                              : work_bytes<double>(net.nB, s.n, net.nPV, s.nblk());
+    return b <= max_lds && s.ch_m <= kBatchChain ? b : 0;
+}
+
+pf_status pf::solve_wg_allow(bool mixed, long long bytes) {
+    BHIP(hipFuncSetAttribute(mixed ? (const void *)k_solve_wg<float> : (const void *)k_solve_wg<double>,
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    return PF_OK;
+}
+
+pf_status pf::launch_solve_wg(const DevNet &N, const DevSym &Y, const DevState &S, int nblk, const pf_options &opt,
+                              bool mixed, long long lds, Ctl *out, hipStream_t st) {
+    BatchTopo tp{};
+    tp.N = N;
+    tp.Y = Y;
+    tp.nslot = Y.nslot;
+    tp.nblk = nblk;
+    BatchJob J{};
+    J.max_iter = opt.no_max_iter;
+    J.lim = opt.lim_inj_reat ? 1 : 0;
+    J.refine = mixed ? opt.refine_steps : 0;
+    J.tol = opt.tolerancia;
+    J.diverge = 0;   // run to max_iter, as the kernels across the GPU do
+    if (mixed) k_solve_wg<float><<<1, 512, (size_t)lds, st>>>(tp, J, S, out);
+    else k_solve_wg<double><<<1, 512, (size_t)lds, st>>>(tp, J, S, out);
+    BHIP(hipGetLastError());
+    return PF_OK;
+}
 
 namespace {
 std::mutex g_scratch_mu;

@@ -171,4 +171,12 @@ inline long long tail_sweep_lds(int nt, int nlev_tail, int nent, bool staged, bo
     return b;
 }
 
+// The whole NR loop in one workgroup (batch.hip): LDS bytes it needs (0: does
+// not run there), the permission for them, and the launch; *out is host
+// memory that the device writes.
+long long solve_wg_lds(const pf_network &net, const Symbolic &s, bool mixed, long long max_lds);
+pf_status solve_wg_allow(bool mixed, long long bytes);
+pf_status launch_solve_wg(const DevNet &N, const DevSym &Y, const DevState &S, int nblk, const pf_options &opt,
+                          bool mixed, long long lds, Ctl *out, hipStream_t st);
+
 }  // namespace pf

@@ -40,6 +40,9 @@ constexpr int kChainMaxF64 = 101;
 // for the batch's LDS-resident topologies, whose 256 threads then hold a
 // block each (118 buses, 333 scenarios, FP64: 18 nodes 809 us, 16 735).
 constexpr int top_width(int m, int pairs_to) { return m <= 16 ? 3 : m <= pairs_to ? 2 : 1; }
+// most nodes of the dense top where one workgroup runs the whole NR loop: one
+// block a thread of its inverse
+constexpr int kSolveWgChain = 22;
 // elimination-tree levels narrower than this run inside one workgroup (the
 // single-network solver's tail); the levels below it form subtree groups
 constexpr int kTailWidth = 64;

@@ -72,6 +72,7 @@ struct pf_solver {
     DevParts dps{};
     int psw_lds[2][2] = {{0, 0}, {0, 0}};
     int flat_ne = 0;
+    long long wg_lds = 0;   // LDS bytes of the loop in one workgroup, 0: across the GPU
     int flat_lds[2] = {0, 0}, parts_lds[2] = {0, 0};
     int flat_cap = 0;   // FP32 tail: most destinations of a step whose blocks the next step reads from LDS
     int tail_mode[2] = {0, 0};
@@ -165,6 +166,7 @@ struct pf_solver {
     template <typename T> pf_status enqueue_solve(const T *blk, double *v, int gate);
     pf_status enqueue_step(int gate);
     pf_status solve(pf_result *r);
+    pf_status outcome(const Ctl &c, std::chrono::steady_clock::time_point t0, pf_result *res) const;
     pf_status run_hybrid_step();
     pf_status ensure_dense();
     pf_status account_pass(bool step, double *pass_ms);
@@ -188,6 +190,17 @@ pf_status pf_solver::build() {
     if (!sym.level_ordered() || (sym.ch_m > 0 && sym.tail_start > sym.nlev_s)) {
         g_last_error = "symbolic analysis: nodes not numbered level by level, or chain outside the tail";
         return PF_INVALID_ARG;
+    }
+    if (opt.lu_blocked && path() == PF_ESPARSO) {   // small networks: the whole loop in one workgroup
+        int max_lds = 0;
+        HIPCHK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+        Symbolic s1 = sym;
+        dense_top(s1, kSolveWgChain, kSolveWgChain);
+        wg_lds = solve_wg_lds(net, s1, mixed(), max_lds - 8192);
+        if (wg_lds) {
+            sym = s1;
+            PFCHK(solve_wg_allow(mixed(), max_lds - 8192));
+        }
     }
     const int nB = net.nB, n = sym.n, sl = net.slack;
     // slot of every Y entry (for the reduced-layout Jacobian export)
@@ -727,6 +740,13 @@ pf_status pf_solver::trace_pass(int pass, const Ctl &c, const double *pass_ms) {
 
 pf_status pf_solver::solve(pf_result *res) {
     HIPCHK(hipSetDevice(device));
+    if (wg_lds && !timing && !trace_cb) {
+        auto t0 = std::chrono::steady_clock::now();
+        ctl_host[0] = Ctl{};
+        PFCHK(launch_solve_wg(dn, dy, ds, sym.nblk(), opt, mixed(), wg_lds, ctl_host, stream));
+        HIPCHK(hipStreamSynchronize(stream));
+        return outcome(ctl_host[0], t0, res);
+    }
     PFCHK(reset_ctl());
     if (timing) {
         const double yb = times.ybus_ms, fl = times.flows_ms;
@@ -796,14 +816,18 @@ pf_status pf_solver::solve(pf_result *res) {
             if (c.done || c.singular) break;
         }
     }
-    auto t1 = std::chrono::steady_clock::now();
-    if (timing) times.iterative_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
+    if (timing)
+        times.iterative_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    return outcome(c, t0, res);
+}
+
+pf_status pf_solver::outcome(const Ctl &c, std::chrono::steady_clock::time_point t0, pf_result *res) const {
     res->iterations = c.it;
     res->converged = c.done && !c.singular;
     res->singular = c.singular;
     res->max_mismatch = c.maxG;
     res->n_switch_events = c.flips;
-    res->solve_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
+    res->solve_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (c.singular) return PF_SINGULAR;
     return res->converged ? PF_OK : PF_NOT_CONVERGED;
 }

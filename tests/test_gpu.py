@@ -406,3 +406,44 @@ def test_lu_solve_dense_tops(pf, synth, tmp_path, copies, precision):
     r = np.zeros(n)
     np.add.at(r, np.repeat(np.arange(n), np.diff(rp)), v * x[cj])
     assert np.abs(r - b).max() <= 1e-9 * np.abs(v).max() * np.abs(x).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("name", ["c14", "ieee57", "c118", "ieee118"])
+def test_nr_one_workgroup(pf, cases, name, precision):
+    """Networks that one CU holds take the whole loop in one workgroup; with stage timing on, the
+    kernels across the GPU run.  Both take the same Newton steps, so after each pass count the
+    states agree to the rounding of the steps: within 1e-9 in FP64, the FP32 factors with one
+    refinement leave about (100 * 6e-8)^2 of a step, 1e-7 after the passes here.
+    """
+    tol = 1e-9 if precision == "fp64" else 1e-7
+    net = pf.Network(_path(cases, name))
+    for lim in (0, 1):
+        for max_iter in (0, 1, 3, 4):
+            both = []
+            for timing in (False, True):
+                s = pf.Solver(net, pf.options(tolerancia=1e-8, no_max_iter=max_iter, lim_inj_reat=lim, refine_steps=1,
+                                              precision=pf.MIXED if precision == "mixed" else pf.FP64))
+                pf.lib().pf_solver_set_timing(s.h, int(timing))
+                r = [s.solve(), s.solve()]          # from the start, and on from where that one ended
+                both.append((r, s.state(), np.concatenate(s.flows())))
+            (ra, sa, fa), (rb, sb, fb) = both
+            for x, y in zip(ra, rb):
+                for k in ("status", "iterations", "converged", "singular", "n_switch_events"):
+                    assert x[k] == y[k], (name, lim, max_iter, k, x, y)
+            assert np.abs(sa[0] - sb[0]).max() <= tol and np.abs(sa[1] - sb[1]).max() <= tol
+            assert np.array_equal(sa[2], sb[2])
+            assert np.abs(fa - fb).max() <= 1e4 * tol     # branch admittances up to some 1e3
+
+
+def test_nr_one_workgroup_singular(pf, cases):
+    """A flat zero voltage has no pivot: both paths say so after the same pass."""
+    net = pf.Network(_path(cases, "c14"))
+    got = []
+    for timing in (False, True):
+        s = pf.Solver(net, pf.options(tolerancia=1e-8, no_max_iter=10))
+        pf.lib().pf_solver_set_timing(s.h, int(timing))
+        s.set_state(np.zeros(net.nB), np.zeros(net.nB))
+        r = s.solve()
+        got.append((r["status"], r["iterations"], r["converged"], r["singular"]))
+    assert got[0] == got[1] and got[0][3]
