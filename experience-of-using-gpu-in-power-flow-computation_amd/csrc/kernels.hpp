@@ -123,7 +123,7 @@ struct DevTail {
 // step, or -1); lv0: the first level of a level-by-level program.
 struct DevFlat {
     int lv0, nsteps, max_pairs, max_col, de_sentinel;
-    const int *fl_ptr, *fl_split, *fl_a, *fl_b, *fl_s, *de_ptr;
+    const int *fl_ptr, *fl_split, *fl_a, *fl_b, *fl_s, *fl_w, *de_ptr;
     const int *de_node, *de_p, *de_q0, *de_ext, *de_lo, *de_hi, *de_dlo, *de_dhi, *de_lr, *st_g;
 };
 

@@ -192,7 +192,7 @@ TailSweeps tail_sweeps(const Symbolic &s);
 //   = the nodes of group g on level l (every pair is inside the group).
 struct FlatTail {
     int lv0 = 0;
-    std::vector<int> fl_ptr, fl_split, fl_a, fl_b, fl_s, de_ptr;
+    std::vector<int> fl_ptr, fl_split, fl_a, fl_b, fl_s, fl_w, de_ptr;
     std::vector<int> de_node, de_p, de_q0, de_ext, de_lo, de_hi, de_dlo, de_dhi, de_lr, st_g;
     int max_pairs = 0, max_col = 0;
     bool stage_ok = true;   // fl_s is usable (a pair's two positions always share a step)

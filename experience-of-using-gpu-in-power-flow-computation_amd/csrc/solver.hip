@@ -461,6 +461,7 @@ pf_status pf_solver::upload_flat(const FlatTail &ft, DevFlat &F) {
     PFCHK(upload((int **)&F.fl_a, ft.fl_a));
     PFCHK(upload((int **)&F.fl_b, ft.fl_b));
     PFCHK(upload((int **)&F.fl_s, ft.fl_s));
+    PFCHK(upload((int **)&F.fl_w, ft.fl_w));
     PFCHK(upload((int **)&F.de_ptr, ft.de_ptr));
     PFCHK(upload((int **)&F.de_node, ft.de_node));
     PFCHK(upload((int **)&F.de_p, ft.de_p));

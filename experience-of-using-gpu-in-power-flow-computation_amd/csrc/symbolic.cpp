@@ -482,7 +482,7 @@ namespace {
 // one level step of a flat program: the destinations of the given nodes,
 // the pivots' pairs first (pairs from sources k < t0 left out)
 void flat_step(const Symbolic &s, FlatTail &f, const int *nodes, int nn, int t0, const std::vector<int> &pcol,
-               std::vector<int> &dlo, std::vector<int> &dhi, std::vector<int> &pos_de) {
+               std::vector<int> &dlo, std::vector<int> &dhi, std::vector<int> &pos_de, std::vector<int> &count) {
     const int base = f.fl_ptr.back();
     for (int pass = 0; pass < 2; pass++) {
         if (pass == 1) f.fl_split.push_back((int)f.fl_a.size() - base);
@@ -516,6 +516,25 @@ void flat_step(const Symbolic &s, FlatTail &f, const int *nodes, int nn, int t0,
     }
     const int np = (int)f.fl_a.size() - base;
     const int E0 = f.de_ptr.back(), E1 = (int)f.de_node.size();
+    // the pairs in the order of their blocks (b, then a as listed): neighbours
+    // read the same block of a source's column and its next ones.  Each keeps
+    // its product's place.
+    std::vector<int> la(f.fl_a.begin() + base, f.fl_a.end()), lb(f.fl_b.begin() + base, f.fl_b.end()), bs;
+    for (int b : lb)
+        if (count[b]++ == 0) bs.push_back(b);
+    std::sort(bs.begin(), bs.end());
+    for (int b : bs) {
+        const int c = count[b];
+        count[b] = (int)f.fl_w.size();
+        f.fl_w.resize(f.fl_w.size() + c);
+    }
+    for (int i = 0; i < np; i++) {
+        const int q = count[lb[i]]++;
+        f.fl_a[q] = la[i];
+        f.fl_b[q] = lb[i];
+        f.fl_w[q] = i;
+    }
+    for (int b : bs) count[b] = 0;
     // pairs whose source is a node of the previous step: the slots of their
     // two positions among that step's destinations
     const int P0 = f.de_ptr.size() >= 2 ? f.de_ptr[f.de_ptr.size() - 2] : E0;
@@ -538,6 +557,7 @@ void flat_seal(FlatTail &f) {
     f.fl_a.push_back(0);
     f.fl_b.push_back(0);
     f.fl_s.push_back(-1);
+    f.fl_w.push_back(0);
     f.de_node.push_back(0);
     f.de_p.push_back(-1);
     f.de_q0.push_back(0);
@@ -563,7 +583,7 @@ FlatTail flat_tail(const Symbolic &s, int lv0, bool split_below, int step_blocks
     f.lv0 = lv0;
     const int t0 = split_below ? s.lvl_ptr[lv0] : 0;
     const std::vector<int> pcol = position_columns(s);
-    std::vector<int> dlo(s.n), dhi(s.n), pos_de(s.nnzL, -1);
+    std::vector<int> dlo(s.n), dhi(s.n), pos_de(s.nnzL, -1), count(s.nnzL, 0);
     f.fl_ptr.assign(1, 0);
     f.de_ptr.assign(1, 0);
     // products of a node's step: one per pair, two for a column destination's
@@ -582,14 +602,14 @@ FlatTail flat_tail(const Symbolic &s, int lv0, bool split_below, int step_blocks
         for (int j = s.lvl_ptr[l]; j < s.lvl_ptr[l + 1]; j++) {
             const long long b = blocks(j);
             if (!nodes.empty() && sum + b > step_blocks) {   // the nodes of a level do not depend on each other
-                flat_step(s, f, nodes.data(), (int)nodes.size(), t0, pcol, dlo, dhi, pos_de);
+                flat_step(s, f, nodes.data(), (int)nodes.size(), t0, pcol, dlo, dhi, pos_de, count);
                 nodes.clear();
                 sum = 0;
             }
             nodes.push_back(j);
             sum += b;
         }
-        flat_step(s, f, nodes.data(), (int)nodes.size(), t0, pcol, dlo, dhi, pos_de);
+        flat_step(s, f, nodes.data(), (int)nodes.size(), t0, pcol, dlo, dhi, pos_de, count);
     }
     flat_seal(f);
     return f;
@@ -599,13 +619,13 @@ FlatTail flat_parts(const Symbolic &s) {
     FlatTail f;
     const int T = s.tail_start;
     const std::vector<int> pcol = position_columns(s);
-    std::vector<int> dlo(s.n), dhi(s.n), pos_de(s.nnzL, -1);
+    std::vector<int> dlo(s.n), dhi(s.n), pos_de(s.nnzL, -1), count(s.nnzL, 0);
     f.fl_ptr.assign(1, 0);
     f.de_ptr.assign(1, 0);
     for (int g = 0; g < s.n_parts; g++)
         for (int l = 0; l < T; l++) {
             const int a = s.part_ptr[(size_t)g * T + l], b = s.part_ptr[(size_t)g * T + l + 1];
-            flat_step(s, f, s.part_nodes.data() + a, b - a, 0, pcol, dlo, dhi, pos_de);
+            flat_step(s, f, s.part_nodes.data() + a, b - a, 0, pcol, dlo, dhi, pos_de, count);
         }
     flat_seal(f);
     return f;
@@ -801,8 +821,9 @@ bool host_flat_factor(const Symbolic &s, const FlatTail &parts, const FlatTail &
                     lb = &stage[8 * sb];
                     ub = &stage[8 * sb + 4];
                 }
-                mul2(&pa[4 * (size_t)e], la, ub);
-                if (e >= ns) mul2(&pu[4 * (size_t)(e - ns)], lb, ua);
+                const int w = f.fl_w[base + e];
+                mul2(&pa[4 * (size_t)w], la, ub);
+                if (w >= ns) mul2(&pu[4 * (size_t)(w - ns)], lb, ua);
             }
             next.assign(8 * (size_t)(f.de_ptr[t + 1] - f.de_ptr[t]), std::nan(""));
             for (int E = f.de_ptr[t]; E < f.de_ptr[t + 1]; E++) {
