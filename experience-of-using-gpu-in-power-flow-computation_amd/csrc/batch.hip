@@ -25,6 +25,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "kernels_decl.hpp"
@@ -42,6 +43,7 @@ struct BatchTopo {
     int nslot;                          // Jacobian slots
     int nblk;                           // factor blocks: slots, row-ordered L, chain inverse
     DevFlat F;                          // flat pair program of the narrow top (F.fl_ptr null: none)
+    int ck_max;                         // without it: most chunks of a level of the narrow top
 };
 
 struct BatchJob {
@@ -72,6 +74,8 @@ constexpr int GL = 16;   // lanes per node in the in-workgroup LU and solves
 constexpr int kBatchChain = 32;
 constexpr int kBatchChainWide = 64;
 template <typename T> constexpr int kBatchTile = 2;   // wider tiles spill in the persistent kernel
+// up to 512 threads (MODE 1): as wide as 64 nodes take, in FP32
+template <typename T, int MAXT> constexpr int kLeanTile = sizeof(T) == 8 ? 2 : MAXT <= 256 ? 4 : 3;
 template <int MODE> constexpr int batch_chain_cap() { return MODE == 2 ? kBatchChain : kBatchChainWide; }
 // levels of at least kWideLevel nodes: a lane group per node; narrower ones:
 // the whole workgroup on the level's destinations.  A constant, not the
@@ -365,7 +369,7 @@ __device__ __forceinline__ void wg_solve(const DevSym &Y, const T *blk, double *
     int pr = -1;
     B4<T> pU{0, 0, 0, 0}, pD{0, 0, 0, 0};
     if (nl > 0) fetch_bwd(nl - 1, pr, pU, pD);
-    if (Y.ch_m > 0) chain_solve<T, GL>(Y, blk, x, s_r);
+    if (Y.ch_m > 0) chain_solve<T, GL>(Y, blk, x, s_r, Y.rs_ptr);
     for (int l = nl - 1; l >= 0; l--) {
         int nr = -1;
         B4<T> nU{0, 0, 0, 0}, nD{0, 0, 0, 0};
@@ -404,266 +408,137 @@ __device__ __forceinline__ void wg_solve(const DevSym &Y, const T *blk, double *
     }
 }
 
-// Sum of the products [lo, hi) of an LDS array in index order (four
-// loads in flight before their additions, which keep the order).
-__device__ __forceinline__ double2 prod_sum_in_order(const double2 *v, int lo, int hi) {
-    double a0 = 0, a1 = 0;
-    int q = lo;
-    for (; q + 4 <= hi; q += 4) {
-        const double2 p0 = v[q], p1 = v[q + 1], p2 = v[q + 2], p3 = v[q + 3];
-        a0 += p0.x; a1 += p0.y;
-        a0 += p1.x; a1 += p1.y;
-        a0 += p2.x; a1 += p2.y;
-        a0 += p3.x; a1 += p3.y;
-    }
-    for (; q < hi; q++) {
-        a0 += v[q].x;
-        a1 += v[q].y;
-    }
-    return make_double2(a0, a1);
-}
+// Row or column pointers of the sweeps in 16 bits in LDS, or, past 65,535
+// entries, where they are in memory.
+struct RowPtr16 {
+    const unsigned short *h;
+    const int *g;
+    bool packed;
+    __device__ __forceinline__ int operator[](int i) const { return packed ? (int)h[i] : g[i]; }
+};
 
 // Forward and backward sweeps whose factor entries are loaded a level
 // ahead (they do not depend on x).  The entries of a level are contiguous
-// (rs_ptr / colptr in node order, nodes numbered level by level).
-//  * Narrow levels (at most kSweepGroupLevel nodes, a constant, so every
-//    launch shape sums alike): 16 lanes per node, lane i taking entries
-//    i, i + 16, ...; its first kSweepAhead entries come from registers
-//    filled during the level before.  One barrier per level.
-//  * Wide levels: one entry per lane, the product L_jk x_k (backward
-//    U_ji x_i) into LDS (prod, `page` at a time), then one thread per node
-//    subtracts its products in entry order (backward: and applies the
-//    inverse pivot after the level's last page).  Two barriers per page.
+// (rs_ptr / colptr in node order, nodes numbered level by level).  A level's
+// width alone says how many lanes a node gets, lane i taking entries i,
+// i + g, ..., so every launch shape sums alike: 16 lanes up to
+// kSweepGroupLevel nodes, 4 up to 4 kSweepGroupLevel (256 threads take either
+// at once), one above.  A node's first kSweepAhead entries a lane come from
+// registers filled during the level before; one barrier per level.  (Wide
+// levels went through LDS, an entry's product a lane and two barriers a page
+// of them: 512 x 1,888 buses 4,230 us, now 4,130; 2,048 x 944 9,790, 9,500.)
 constexpr int kSweepGroupLevel = 16, kSweepAhead = 2;
 
-template <typename T>
-__device__ __forceinline__ void wg_solve_flat(const DevSym &Y, const T *blk, double *x, double *s_r, double2 *prod,
-                                              int page) {
-    const int tid = (int)threadIdx.x, bd = (int)blockDim.x, grp = tid / GL, lane = tid % GL;
-    const int LR0 = Y.n + 2 * Y.nnzL, U0 = Y.n + Y.nnzL, nl = Y.nlev_s;
+// one direction: ptr, idx, B0: the rows and L by rows, or the columns and U
+// (BWD, where the sum also meets the node's inverse pivot)
+template <typename T, bool BWD, typename PTR>
+__device__ __forceinline__ void wg_sweep(const DevSym &Y, const T *blk, double *x, const PTR ptr, const int *idx, int B0,
+                                         int nl) {
+    const int tid = (int)threadIdx.x, bd = (int)blockDim.x;
     constexpr int RA = kSweepAhead;
     int pk[RA];
     B4<T> pB[RA], pD{0, 0, 0, 0};
-    int ns = 0, nc = 0, ne0 = 0, ne1 = 0;   // the coming level's first node and width, this lane's node's entries
-    // the entries this lane takes first on level l: a narrow level's node
-    // grp (entries lane + GL r), a wide level's entry tid; ptr / idx / B0 are
-    // the row (forward) or column (backward) structure and its blocks.  The
-    // level's bounds and the node's entry range stay in registers for the
-    // level itself, which then starts with no metadata read.
-    auto ahead = [&](int l, const int *ptr, const int *idx, int B0, bool diag) __attribute__((always_inline)) {
-        const int s = Y.lvl_ptr[l], c = Y.lvl_ptr[l + 1] - s;
-        ns = s;
-        nc = c;
+    // the coming level: its first node and width, log2 of its lanes a node,
+    // the entries of this lane's node (from this lane's first on)
+    int ns = 0, nc = 0, ng = 0, ne = 0, ne1 = 0;
+    auto level = [&](int i) __attribute__((always_inline)) { return BWD ? nl - 1 - i : i; };
+    auto ahead = [&](int l) __attribute__((always_inline)) {
+        ns = Y.lvl_ptr[l];
+        nc = Y.lvl_ptr[l + 1] - ns;
+        ng = nc <= kSweepGroupLevel ? 4 : nc <= 4 * kSweepGroupLevel ? 2 : 0;
+        const int me = tid >> ng, lane = tid & ((1 << ng) - 1);
 #pragma unroll
         for (int r = 0; r < RA; r++) pk[r] = -1;
-        if (c <= kSweepGroupLevel) {
-            if (grp < c) {
-                const int j = s + grp, e1 = ptr[j + 1];
-                ne0 = ptr[j];
-                ne1 = e1;
+        if (me < nc) {
+            const int j = ns + me;
+            ne = ptr[j] + lane;
+            ne1 = ptr[j + 1];
 #pragma unroll
-                for (int r = 0; r < RA; r++) {
-                    const int e = ptr[j] + lane + GL * r;
-                    if (e < e1) {
-                        pk[r] = idx[e];
-                        pB[r] = load_b4(blk, B0 + e);
-                    }
+            for (int r = 0; r < RA; r++) {
+                const int e = ne + (r << ng);
+                if (e < ne1) {
+                    pk[r] = idx[e];
+                    pB[r] = load_b4(blk, B0 + e);
                 }
-                if (diag && lane == 0) pD = load_b4(blk, Y.di0 + j);
             }
-        } else {
-            const int e = ptr[s] + tid;
-            if (e < ptr[s + c]) {
-                pk[0] = idx[e];
-                pB[0] = load_b4(blk, B0 + e);
-            }
-            if (diag && tid < c) pD = load_b4(blk, Y.di0 + s + tid);
+            if (BWD && lane == 0) pD = load_b4(blk, Y.di0 + j);
         }
     };
-    // ---- forward
-    if (nl > 0) ahead(0, Y.rs_ptr, Y.rs_k, LR0, false);
-    for (int l = 0; l < nl; l++) {
-        const int s = ns, c = nc, je0 = ne0, je1 = ne1;
+    auto put = [&](int j, double y0, double y1, const B4<T> &D) __attribute__((always_inline)) {
+        if (BWD) {
+            x[2 * j] = (double)D.a * y0 + (double)D.b * y1;
+            x[2 * j + 1] = (double)D.c * y0 + (double)D.d * y1;
+        } else {
+            x[2 * j] = y0;
+            x[2 * j + 1] = y1;
+        }
+    };
+    if (nl > 0) ahead(level(0));
+    for (int i = 0; i < nl; i++) {
+        const int s = ns, c = nc, sh = ng, e0 = ne, e1 = ne1;
+        const int me = tid >> sh, lane = tid & ((1 << sh) - 1);
         int ck[RA];
         B4<T> cB[RA];
+        double xk[RA][2];   // x of the first entries, read before the next level's requests
 #pragma unroll
         for (int r = 0; r < RA; r++) {
             ck[r] = pk[r];
             cB[r] = pB[r];
+            const int k = ck[r] >= 0 ? ck[r] : 0;
+            xk[r][0] = x[2 * k];
+            xk[r][1] = x[2 * k + 1];
         }
-        if (c <= kSweepGroupLevel) {
-            double xk[RA][2];   // x of the first entries, read before the next level's requests
+        const B4<T> myD = pD;
+        // the node's own x: no earlier level of this sweep writes it
+        const int jo = s + (me < c ? me : 0);
+        const double xj0 = x[2 * jo], xj1 = x[2 * jo + 1];
+        if (i + 1 < nl) ahead(level(i + 1));
+        if (me < c) {
+            double a0 = 0, a1 = 0;
 #pragma unroll
-            for (int r = 0; r < RA; r++) {
-                const int k = ck[r] >= 0 ? ck[r] : 0;
-                xk[r][0] = x[2 * k];
-                xk[r][1] = x[2 * k + 1];
-            }
-            // the node's own x: no earlier level of this sweep writes it
-            const int jo = s + (grp < c ? grp : 0);
-            const double xj0 = x[2 * jo], xj1 = x[2 * jo + 1];
-            if (l + 1 < nl) ahead(l + 1, Y.rs_ptr, Y.rs_k, LR0, false);
-            if (grp < c) {
-                const int j = s + grp;
-                double a0 = 0, a1 = 0;
-#pragma unroll
-                for (int r = 0; r < RA; r++)
-                    if (ck[r] >= 0) {
-                        const double x0 = xk[r][0], x1 = xk[r][1];
-                        a0 += (double)cB[r].a * x0 + (double)cB[r].b * x1;
-                        a1 += (double)cB[r].c * x0 + (double)cB[r].d * x1;
-                    }
-                for (int e = je0 + lane + GL * RA; e < je1; e += GL) {
-                    const B4<T> L = load_b4(blk, LR0 + e);
-                    const int k = Y.rs_k[e];
-                    const double x0 = x[2 * k], x1 = x[2 * k + 1];
-                    a0 += (double)L.a * x0 + (double)L.b * x1;
-                    a1 += (double)L.c * x0 + (double)L.d * x1;
+            for (int r = 0; r < RA; r++)
+                if (ck[r] >= 0) {
+                    a0 += (double)cB[r].a * xk[r][0] + (double)cB[r].b * xk[r][1];
+                    a1 += (double)cB[r].c * xk[r][0] + (double)cB[r].d * xk[r][1];
                 }
-                a0 = xor_sum<GL>(a0);
-                a1 = xor_sum<GL>(a1);
-                if (lane == 0) {
-                    x[2 * j] = xj0 - a0;
-                    x[2 * j + 1] = xj1 - a1;
-                }
-            }
-            __syncthreads();
-            continue;
-        }
-        const int e_lo = Y.rs_ptr[s], e_hi = Y.rs_ptr[s + c];
-        if (e_lo == e_hi && l + 1 < nl) ahead(l + 1, Y.rs_ptr, Y.rs_k, LR0, false);
-        for (int pg = e_lo; pg < e_hi; pg += page) {
-            const int pe = min(pg + page, e_hi);
-            for (int e = pg + tid; e < pe; e += bd) {
-                int k;
-                B4<T> L;
-                if (e == e_lo + tid) {
-                    k = ck[0];
-                    L = cB[0];
-                } else {
-                    k = Y.rs_k[e];
-                    L = load_b4(blk, LR0 + e);
-                }
+            for (int e = e0 + (RA << sh); e < e1; e += 1 << sh) {
+                const B4<T> L = load_b4(blk, B0 + e);
+                const int k = idx[e];
                 const double x0 = x[2 * k], x1 = x[2 * k + 1];
-                prod[e - pg] = make_double2((double)L.a * x0 + (double)L.b * x1, (double)L.c * x0 + (double)L.d * x1);
+                a0 += (double)L.a * x0 + (double)L.b * x1;
+                a1 += (double)L.c * x0 + (double)L.d * x1;
             }
-            if (pg == e_lo && l + 1 < nl) ahead(l + 1, Y.rs_ptr, Y.rs_k, LR0, false);
-            __syncthreads();
-            for (int i = tid; i < c; i += bd) {
-                const int j = s + i, lo = max(Y.rs_ptr[j], pg), hi = min(Y.rs_ptr[j + 1], pe);
-                if (lo < hi) {
-                    const double2 a = prod_sum_in_order(prod, lo - pg, hi - pg);
-                    x[2 * j] -= a.x;
-                    x[2 * j + 1] -= a.y;
-                }
-            }
-            __syncthreads();
-        }
-    }
-    if (Y.ch_m > 0) chain_solve<T, GL>(Y, blk, x, s_r);
-    // ---- backward
-    if (nl > 0) ahead(nl - 1, Y.colptr, Y.rowind, U0, true);
-    for (int l = nl - 1; l >= 0; l--) {
-        const int s = ns, c = nc, je0 = ne0, je1 = ne1;
-        int ck[RA];
-        B4<T> cB[RA];
-#pragma unroll
-        for (int r = 0; r < RA; r++) {
-            ck[r] = pk[r];
-            cB[r] = pB[r];
-        }
-        const B4<T> myD = pD;   // narrow: the inverse pivot of node s + grp (lane 0); wide: of node s + tid
-        if (c <= kSweepGroupLevel) {
-            double xk[RA][2];   // x of the first entries, read before the next level's requests
-#pragma unroll
-            for (int r = 0; r < RA; r++) {
-                const int k = ck[r] >= 0 ? ck[r] : 0;
-                xk[r][0] = x[2 * k];
-                xk[r][1] = x[2 * k + 1];
-            }
-            // the node's own x: no earlier level of this sweep writes it
-            const int jo = s + (grp < c ? grp : 0);
-            const double xj0 = x[2 * jo], xj1 = x[2 * jo + 1];
-            if (l > 0) ahead(l - 1, Y.colptr, Y.rowind, U0, true);
-            if (grp < c) {
-                const int j = s + grp;
-                double a0 = 0, a1 = 0;
-#pragma unroll
-                for (int r = 0; r < RA; r++)
-                    if (ck[r] >= 0) {
-                        const double x0 = xk[r][0], x1 = xk[r][1];
-                        a0 += (double)cB[r].a * x0 + (double)cB[r].b * x1;
-                        a1 += (double)cB[r].c * x0 + (double)cB[r].d * x1;
-                    }
-                for (int e = je0 + lane + GL * RA; e < je1; e += GL) {
-                    const B4<T> U = load_b4(blk, U0 + e);
-                    const int i = Y.rowind[e];
-                    const double x0 = x[2 * i], x1 = x[2 * i + 1];
-                    a0 += (double)U.a * x0 + (double)U.b * x1;
-                    a1 += (double)U.c * x0 + (double)U.d * x1;
-                }
+            if (sh == 4) {
                 a0 = xor_sum<GL>(a0);
                 a1 = xor_sum<GL>(a1);
-                if (lane == 0) {
-                    const double y0 = xj0 - a0, y1 = xj1 - a1;
-                    x[2 * j] = (double)myD.a * y0 + (double)myD.b * y1;
-                    x[2 * j + 1] = (double)myD.c * y0 + (double)myD.d * y1;
-                }
+            } else if (sh == 2) {
+                a0 = quad_sum(a0);
+                a1 = quad_sum(a1);
             }
-            __syncthreads();
-            continue;
+            if (lane == 0) put(jo, xj0 - a0, xj1 - a1, myD);
+            if (sh == 0)
+                for (int j = s + me + bd; j < s + c; j += bd) {
+                    double b0 = 0, b1 = 0;
+                    for (int e = ptr[j], ee = ptr[j + 1]; e < ee; e++) {
+                        const B4<T> L = load_b4(blk, B0 + e);
+                        const int k = idx[e];
+                        const double x0 = x[2 * k], x1 = x[2 * k + 1];
+                        b0 += (double)L.a * x0 + (double)L.b * x1;
+                        b1 += (double)L.c * x0 + (double)L.d * x1;
+                    }
+                    put(j, x[2 * j] - b0, x[2 * j + 1] - b1, BWD ? load_b4(blk, Y.di0 + j) : B4<T>{0, 0, 0, 0});
+                }
         }
-        const int e_lo = Y.colptr[s], e_hi = Y.colptr[s + c];
-        if (e_lo == e_hi) {     // no entries: only the inverse pivots
-            if (l > 0) ahead(l - 1, Y.colptr, Y.rowind, U0, true);
-            for (int i = tid; i < c; i += bd) {
-                const int j = s + i;
-                const B4<T> D = (i == tid) ? myD : load_b4(blk, Y.di0 + j);
-                const double y0 = x[2 * j], y1 = x[2 * j + 1];
-                x[2 * j] = (double)D.a * y0 + (double)D.b * y1;
-                x[2 * j + 1] = (double)D.c * y0 + (double)D.d * y1;
-            }
-            __syncthreads();
-            continue;
-        }
-        for (int pg = e_lo; pg < e_hi; pg += page) {
-            const int pe = min(pg + page, e_hi);
-            for (int e = pg + tid; e < pe; e += bd) {
-                int r;
-                B4<T> U;
-                if (e == e_lo + tid) {
-                    r = ck[0];
-                    U = cB[0];
-                } else {
-                    r = Y.rowind[e];
-                    U = load_b4(blk, U0 + e);
-                }
-                const double x0 = x[2 * r], x1 = x[2 * r + 1];
-                prod[e - pg] = make_double2((double)U.a * x0 + (double)U.b * x1, (double)U.c * x0 + (double)U.d * x1);
-            }
-            if (pg == e_lo && l > 0) ahead(l - 1, Y.colptr, Y.rowind, U0, true);
-            __syncthreads();
-            const bool last = pe == e_hi;
-            for (int i = tid; i < c; i += bd) {
-                const int j = s + i, lo = max(Y.colptr[j], pg), hi = min(Y.colptr[j + 1], pe);
-                double y0 = x[2 * j], y1 = x[2 * j + 1];
-                if (lo < hi) {
-                    const double2 a = prod_sum_in_order(prod, lo - pg, hi - pg);
-                    y0 -= a.x;
-                    y1 -= a.y;
-                }
-                if (last) {
-                    const B4<T> D = (i == tid) ? myD : load_b4(blk, Y.di0 + j);
-                    x[2 * j] = (double)D.a * y0 + (double)D.b * y1;
-                    x[2 * j + 1] = (double)D.c * y0 + (double)D.d * y1;
-                } else if (lo < hi) {
-                    x[2 * j] = y0;
-                    x[2 * j + 1] = y1;
-                }
-            }
-            __syncthreads();
-        }
+        __syncthreads();
     }
+}
+
+template <typename T, typename PTR>
+__device__ __forceinline__ void wg_solve_flat(const DevSym &Y, const T *blk, double *x, double *s_r, const PTR rs,
+                                              const PTR cl) {
+    wg_sweep<T, false>(Y, blk, x, rs, Y.rs_k, Y.n + 2 * Y.nnzL, Y.nlev_s);
+    if (Y.ch_m > 0) chain_solve<T, GL>(Y, blk, x, s_r, rs);
+    wg_sweep<T, true>(Y, blk, x, cl, Y.rowind, Y.n + Y.nnzL, Y.nlev_s);
 }
 
 // I = Y E and S = E conj(I): 4 lanes per row
@@ -825,10 +700,14 @@ __device__ __forceinline__ void wg_start(const BatchTopo &tp, Work<T> &w, const 
 // One NR solve of one scenario by the whole workgroup from the state in w.
 // Returns (via shared result) iterations, converged flag, final max mismatch,
 // flips and whether a pivot failed (s_end, may be null).
-template <typename T>
+// s_chain: LDS of the dense top and of a narrow level's pivots; s_ck: of the
+// chunked narrow top, null: the working set is in LDS; rs, cl: row and column
+// pointers of the flat sweeps.
+template <typename T, int TMAX, typename PTR>
 __device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Work<T> &w, const double *Pliq,
                       const double *Qliq, const double *Qload,
-                      int *s_it, int *s_conv, double *s_maxg, int *s_fl, int *s_end, B4<T> *s_chain, B4<T> *s_ck) {
+                      int *s_it, int *s_conv, double *s_maxg, int *s_fl, int *s_end, B4<T> *s_chain, B4<T> *s_ck, int ck_max,
+                      const PTR rs, const PTR cl) {
     const DevNet &N = tp.N;
     const DevSym &Y = tp.Y;
     __shared__ unsigned long long s_maxG_bits, s_maxDx_bits;
@@ -959,7 +838,7 @@ __device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Wo
                 }
                 if (s_ck && Y.ck_lvl && l >= Y.tail_start) {   // the chunked narrow top
                     chunk_factor_levels<T, kBatchChunkLanes, 1>(Y, w.blk, l, Y.nlev_s, &s_sing, s_ck,
-                                                                  s_ck + kBatchMaxChunks, s_chain);
+                                                                  s_ck + ck_max, s_chain);
                     break;
                 }
                 const int s = Y.lvl_ptr[l], c = Y.lvl_ptr[l + 1] - s;
@@ -975,21 +854,19 @@ __device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Wo
                 }
             }
             if (Y.ch_m > 0) {
-                chain_factor_mem<T, GL, kBatchUnroll, kBatchTile<T>>(Y, w.blk, &s_sing, s_chain);
+                chain_factor_mem<T, GL, kBatchUnroll, TMAX>(Y, w.blk, &s_sing, s_chain);
                 __syncthreads();
             }
         }
         if (s_sing) break;
         for (int i = tid; i < 2 * Y.n; i += blockDim.x) w.x[i] = w.g[i];
         __syncthreads();
-        // the flat sweeps take their products in s_ck (free after the factorisation)
-        const int page = (int)(sizeof(B4<T>) * 2 * kBatchMaxChunks / sizeof(double2));
-        if (s_ck) wg_solve_flat(Y, (const T *)w.blk, w.x, (double *)s_chain, reinterpret_cast<double2 *>(s_ck), page);
+        if (s_ck) wg_solve_flat(Y, (const T *)w.blk, w.x, (double *)s_chain, rs, cl);
         else wg_solve(Y, (const T *)w.blk, w.x, (double *)s_chain);
-        for (int rs = 0; rs < J.refine; rs++) {
+        for (int q = 0; q < J.refine; q++) {
             wg_residual(N, w);
             __syncthreads();
-            if (s_ck) wg_solve_flat(Y, (const T *)w.blk, w.r, (double *)s_chain, reinterpret_cast<double2 *>(s_ck), page);
+            if (s_ck) wg_solve_flat(Y, (const T *)w.blk, w.r, (double *)s_chain, rs, cl);
             else wg_solve(Y, (const T *)w.blk, w.r, (double *)s_chain);
             for (int i = tid; i < 2 * Y.n; i += blockDim.x) w.x[i] += w.r[i];
             __syncthreads();
@@ -1040,6 +917,30 @@ __host__ __device__ inline long long partial_lds_bytes(int n, int nlev) {
     return (b + 255) & ~255LL;
 }
 
+// blocks of LDS of the dense top, or of a narrow level's pivots
+__host__ __device__ inline int chain_lds_blocks(int ch_m) {
+    return 4 * ch_m + 2 > kWideLevel ? 4 * ch_m + 2 : kWideLevel;
+}
+
+// LDS of MODE 1 up to 512 threads, where several workgroups share a CU: the
+// step vectors x and r, the dense top's staging, the level pointers and,
+// packed, the row and column pointers, and the partial sums of a chunked
+// narrow top.  The rest of MODE 1's arrays is read where it is in memory.
+template <typename T>
+struct LeanLds {
+    long long buf, ck, lvl, rs, cl, bytes;   // offsets, and the whole
+    bool packed;
+    __host__ __device__ LeanLds(int n, int nnzL, int nlev, int ch_m, int chunks) {
+        buf = 32LL * n;
+        ck = buf + (long long)sizeof(B4<T>) * chain_lds_blocks(ch_m);
+        lvl = ck + (long long)sizeof(B4<T>) * 2 * chunks;
+        rs = lvl + 4LL * (nlev + 1);
+        packed = nnzL <= 65535;
+        cl = rs + (packed ? 2LL * (n + 1) : 0);
+        bytes = (cl + (packed ? 2LL * (n + 1) : 0) + 255) & ~255LL;
+    }
+};
+
 // MODE 2: the whole per-scenario working set in LDS.
 // MODE 1: working set in a global slice, except the step vectors and the
 //         level / row-structure metadata, staged in LDS (latency of the
@@ -1047,21 +948,52 @@ __host__ __device__ inline long long partial_lds_bytes(int n, int nlev) {
 // The float LDS-resident kernel at 256 threads keeps three waves per SIMD
 // (three workgroups per CU, within 168 VGPRs): small networks are latency
 // bound, so more resident scenarios per CU beat the few registers it costs.
+// MODE 1 keeps four (128 VGPRs) at every size, so that two workgroups of 512
+// or four of 256 share a CU, and up to 512 threads it takes less LDS for it
+// (LeanLds: x, r and 16-bit pointers; g in the slice).  A pass waits on loads
+// and barriers, which one workgroup alone does not cover: 2,048 x 944 buses in
+// FP32 9,840 us one of 1024, 7,090 two of 512; 2,048 x 354 buses 3,070 us two
+// of 256 at 183 VGPRs, 2,090 four at 128.
 template <typename T, int MODE, int MAXT>
-constexpr int batch_min_waves() { return (MODE == 2 && MAXT == 256 && sizeof(T) == 4) ? 3 : 1; }
+constexpr int batch_min_waves() { return MODE == 1 ? 4 : (MODE == 2 && MAXT == 256 && sizeof(T) == 4) ? 3 : 1; }
 
 template <typename T, int MODE, int MAXT>   // MAXT: largest workgroup (register budget)
 __global__ void __launch_bounds__(MAXT, (batch_min_waves<T, MODE, MAXT>())) k_batch(BatchTopo tp0, BatchJob J) {
     extern __shared__ __align__(16) char smem[];
     __shared__ int s_item, s_it, s_conv, s_fl;
-    __shared__ B4<T> s_chain[4 * batch_chain_cap<MODE>() + 2];   // dense top: row / column / pivot staging
-    __shared__ B4<T> s_ck[MODE == 2 ? 1 : 2 * kBatchMaxChunks];  // chunk partial sums (a, u)
+    constexpr bool lean = MODE == 1 && MAXT < 1024;                // its buffers are in smem (LeanLds)
+    __shared__ B4<T> s_chain_own[lean ? 1 : 4 * batch_chain_cap<MODE>() + 2];   // dense top: row / column / pivot staging
+    __shared__ B4<T> s_ck_own[lean || MODE == 2 ? 1 : 2 * kBatchMaxChunks];     // chunk partial sums (a, u)
     __shared__ double s_maxg;
+    B4<T> *s_chain = s_chain_own, *s_ck = MODE == 2 ? nullptr : s_ck_own;
+    const int ck_max = lean ? tp0.ck_max : kBatchMaxChunks;
     BatchTopo tp = tp0;
     const DevNet &N = tp.N;
     char *base = (MODE == 2) ? smem : J.gws + (long long)blockIdx.x * J.ws_bytes;
     Work<T> w = carve<T>(base, N.nB, tp.Y.n, N.nPV, tp.nblk);
-    if (MODE == 1) {
+    using Ptr = std::conditional_t<lean, RowPtr16, const int *>;
+    Ptr rs, cl;
+    if constexpr (lean) {
+        const int n = tp.Y.n, nlev = tp.Y.nlev;
+        const LeanLds<T> o(n, tp.Y.nnzL, nlev, tp.Y.ch_m, tp.ck_max);
+        w.x = reinterpret_cast<double *>(smem);
+        w.r = w.x + 2 * n;
+        s_chain = reinterpret_cast<B4<T> *>(smem + o.buf);
+        s_ck = reinterpret_cast<B4<T> *>(smem + o.ck);
+        int *lvl = reinterpret_cast<int *>(smem + o.lvl);
+        for (int i = threadIdx.x; i <= nlev; i += blockDim.x) lvl[i] = tp0.Y.lvl_ptr[i];
+        tp.Y.lvl_ptr = lvl;
+        unsigned short *r16 = reinterpret_cast<unsigned short *>(smem + o.rs);
+        unsigned short *c16 = reinterpret_cast<unsigned short *>(smem + o.cl);
+        if (o.packed)
+            for (int i = threadIdx.x; i <= n; i += blockDim.x) {
+                r16[i] = (unsigned short)tp0.Y.rs_ptr[i];
+                c16[i] = (unsigned short)tp0.Y.colptr[i];
+            }
+        rs = RowPtr16{r16, tp0.Y.rs_ptr, o.packed};
+        cl = RowPtr16{c16, tp0.Y.colptr, o.packed};
+        __syncthreads();
+    } else if constexpr (MODE == 1) {
         const int n = tp.Y.n, nlev = tp.Y.nlev;
         double *v = reinterpret_cast<double *>(smem);
         w.g = v;
@@ -1081,6 +1013,10 @@ __global__ void __launch_bounds__(MAXT, (batch_min_waves<T, MODE, MAXT>())) k_ba
         tp.Y.fd_ptr = stage(tp0.Y.fd_ptr, n + 1);
         __syncthreads();
     }
+    if constexpr (!lean) {
+        rs = tp.Y.rs_ptr;
+        cl = tp.Y.colptr;
+    }
     const int nscen = J.nscen_dev ? *J.nscen_dev : J.nscen;
     for (;;) {
         if (threadIdx.x == 0) s_item = atomicAdd(J.counter, 1);
@@ -1098,8 +1034,8 @@ __global__ void __launch_bounds__(MAXT, (batch_min_waves<T, MODE, MAXT>())) k_ba
         for (int attempt = warm ? 0 : 1; attempt < 2; ++attempt) {
             const bool from_warm = attempt == 0;
             wg_start(tp, w, Ql, from_warm ? J.V0 + off : tp.V0flat, from_warm ? J.th0 + off : tp.th0flat);
-            wg_nr(tp, J, w, Pl, Ql, Qd, &s_it, &s_conv, &s_maxg, &s_fl, (int *)nullptr, s_chain,
-                  MODE == 2 ? nullptr : s_ck);
+            wg_nr<T, lean ? kLeanTile<T, MAXT> : kBatchTile<T>>(tp, J, w, Pl, Ql, Qd, &s_it, &s_conv, &s_maxg, &s_fl,
+                                                                (int *)nullptr, s_chain, s_ck, ck_max, rs, cl);
             total_it += s_it;
             if (s_conv) break;                              // shared: uniform over the workgroup
         }
@@ -1144,7 +1080,8 @@ __global__ void __launch_bounds__(512) k_solve_wg(BatchTopo tp, BatchJob J, DevS
         w.isq[k] = S.isq[k];
     }
     for (int i = threadIdx.x; i < N.nPV; i += blockDim.x) w.limQ[i] = S.limQ[i];
-    wg_nr(tp, J, w, S.Pliq, S.Qliq, S.Qload, &s_it, &s_conv, &s_maxg, &s_fl, &s_end, s_chain, (B4<T> *)nullptr);
+    wg_nr<T, kBatchTile<T>>(tp, J, w, S.Pliq, S.Qliq, S.Qload, &s_it, &s_conv, &s_maxg, &s_fl, &s_end, s_chain,
+                            (B4<T> *)nullptr, 0, tp.Y.rs_ptr, tp.Y.colptr);
     for (int k = threadIdx.x; k < N.nB; k += blockDim.x) {
         S.V[k] = w.V[k];
         S.th[k] = w.th[k];
@@ -1422,6 +1359,7 @@ struct pf_batch {
     pf_status launch_net(size_t i, hipStream_t s);
     pf_status launch_all();
     pf_status configure(BatchNet &nb, int mode, int block, int per_cu);
+    long long shm_bytes(const BatchNet &nb, int mode, int block) const;
     pf_status occupancy(BatchNet &nb, int mode, int block, int *per_cu);
     pf_status default_shape(BatchNet &nb, int nscen, int *block, int *per_cu);
     void drop_graph() {
@@ -1562,6 +1500,7 @@ pf_status pf_batch::add_net(const pf_network &src) {
     }
     BCHK(upload((double **)&b->tp.V0flat, net.V));
     BCHK(upload((double **)&b->tp.th0flat, net.theta));
+    b->tp.ck_max = Y.ck_lvl && !b->tp.F.fl_ptr ? sym.ck_max : 0;
     b->tp.nslot = sym.nslot();
     b->tp.nblk = sym.nblk();
     k_ybus<<<(yp.nnz + 255) / 256, 256, 0, st[0]>>>(N, yp.nnz);
@@ -1586,7 +1525,8 @@ pf_status pf_batch::add_net(const pf_network &src) {
             for (int blk : {256, 512, 1024})
                 if (e == hipSuccess)
                     e = hipFuncSetAttribute((const void *)batch_kernel(mixed, 1, blk),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)pb);
+                                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (int)(blk > 512 ? pb : max_lds));
         if (pb <= max_lds && e == hipSuccess) {
             b->partial = pb;
             b->mode = 1;
@@ -1602,6 +1542,16 @@ pf_status pf_batch::add_net(const pf_network &src) {
     return PF_OK;
 }
 
+// dynamic LDS of k_batch<T, mode> at this block size
+long long pf_batch::shm_bytes(const BatchNet &nb, int mode, int block) const {
+    if (mode != 1) return mode == 2 ? nb.ws : 0;
+    if (block > 512) return nb.partial;
+    const Symbolic &y = nb.sym;
+    const int ck = nb.tp.ck_max;
+    return opt.precision != PF_FP64 ? LeanLds<float>(y.n, y.nnzL, y.nlev, y.ch_m, ck).bytes
+                                    : LeanLds<double>(y.n, y.nnzL, y.nlev, y.ch_m, ck).bytes;
+}
+
 // resident workgroups per CU of k_batch<T, mode> at this block size
 pf_status pf_batch::occupancy(BatchNet &nb, int mode, int block, int *per_cu) {
     int &known = nb.occ[mode][block / 64];
@@ -1610,7 +1560,7 @@ pf_status pf_batch::occupancy(BatchNet &nb, int mode, int block, int *per_cu) {
         return PF_OK;
     }
     const bool mixed = opt.precision != PF_FP64;
-    const size_t shm = mode == 2 ? (size_t)nb.ws : mode == 1 ? (size_t)nb.partial : 0;
+    const size_t shm = (size_t)shm_bytes(nb, mode, block);
     int pc = 0;
     BHIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc, (const void *)batch_kernel(mixed, mode, block), block,
                                                       shm));
@@ -1627,10 +1577,16 @@ pf_status pf_batch::occupancy(BatchNet &nb, int mode, int block, int *per_cu) {
 //   LDS (MODE 2): 512 threads up to one scenario per CU, 256 above; up to 64
 //   nodes and more scenarios than fit at once, 128 (57 buses, FP32, 1,500
 //   scenarios: 463 -> 339 us).
-//   MODE 1 / 0: 1024 threads, one per CU; up to kNarrowNodes nodes and more
-//   scenarios than CUs, two of 256 (354 buses, FP64, 1,500 scenarios: 6.11
-//   -> 4.51 ms; on 590 buses 15.8 -> 18.9, so not there).
-constexpr int kNarrowNodes = 400;
+//   MODE 1 / 0: 1024 threads, one per CU, up to one scenario per CU.  With
+//   more, in MODE 1, two of 512 as long as a slice of global workspace stays
+//   within kSlicePair: beyond, 512 of them are so far out of the 256 MB
+//   Infinity Cache that nothing is gained (1,024 scenarios, FP32: 472 buses
+//   2,410 -> 1,690 us, 944 4,580 -> 3,550, 1,416 5,920 -> 5,190, 1,888 (716 KB)
+//   7,800 -> 7,640; FP64: 708 buses 3,740 -> 3,260, 1,180 6,920 -> 6,780, 1,416
+//   8,740 -> 8,860); with more than two per CU, four of 256 where they fit,
+//   up to kSliceQuad (FP32: 354 buses 1,390 -> 1,070, 708 2,160 -> 1,970, 944
+//   3,550 -> 3,650; FP64: 354 buses 1,650 -> 1,420, 472 2,190 -> 2,100).
+constexpr long long kSlicePair = 768 * 1024, kSliceQuad = 320 * 1024;
 pf_status pf_batch::default_shape(BatchNet &nb, int nscen, int *block, int *per_cu) {
     int occ = 0;
     if (nb.mode == 2) {
@@ -1645,10 +1601,19 @@ pf_status pf_batch::default_shape(BatchNet &nb, int nscen, int *block, int *per_
     }
     *block = 1024;
     *per_cu = 1;
-    if (nscen > cus && nb.sym.n <= kNarrowNodes) {
-        BCHK(occupancy(nb, nb.mode, 256, &occ));
-        if (occ >= 2) {
+    if (nb.mode != 1 || nscen <= cus) return PF_OK;
+    if (nscen > 2 * cus && nb.ws <= kSliceQuad) {
+        BCHK(occupancy(nb, 1, 256, &occ));
+        if (occ >= 4) {
             *block = 256;
+            *per_cu = 4;
+            return PF_OK;
+        }
+    }
+    if (nb.ws <= kSlicePair) {
+        BCHK(occupancy(nb, 1, 512, &occ));
+        if (occ >= 2) {
+            *block = 512;
             *per_cu = 2;
         }
     }
@@ -1676,7 +1641,7 @@ pf_status pf_batch::configure(BatchNet &nb, int mode, int block, int per_cu) {
     nb.mode = mode;
     nb.block = block;
     nb.per_cu = per_cu;
-    nb.shm = mode == 2 ? nb.ws : mode == 1 ? nb.partial : 0;
+    nb.shm = shm_bytes(nb, mode, block);
     nb.grid = std::max(1, std::min<int>((int)nb.scen.size(), per_cu * cus));
     if (mode != 2) {
         const size_t need = (size_t)nb.grid * (size_t)nb.ws;
@@ -1996,6 +1961,7 @@ pf_status pf_batch_autotune(pf_batch *b, const char *cache_path, int reps, int *
                     if (b->occupancy(nb, mode, block, &occ) != PF_OK || occ < 1) continue;
                     cands.push_back({mode, block, 1});
                     if (occ >= 2) cands.push_back({mode, block, 2});
+                    if (occ >= 4) cands.push_back({mode, block, 4});
                 }
             }
         }
@@ -2115,7 +2081,10 @@ extern "C" pf_status pf_batch_solve_noalloc(pf_batch *b, int n_scen, const int *
     for (int i = 0; i < nn; i++) {
         BatchNet &nb = *b->nets[i];
         int block = nb.block, per_cu = nb.per_cu;
-        if (nb.grid == 0) BCHK(b->default_shape(nb, n_scen, &block, &per_cu));
+        if (nb.grid == 0) {   // the shape for as many scenarios as have a slice
+            const long long fit = nb.mode == 2 ? n_scen : std::min<long long>(n_scen, share / nb.ws);
+            BCHK(b->default_shape(nb, (int)fit, &block, &per_cu));
+        }
         int grid = std::max(1, per_cu * b->cus);
         if (nb.mode != 2) {
             grid = (int)std::min<long long>(grid, share / nb.ws);
@@ -2167,7 +2136,7 @@ extern "C" pf_status pf_batch_solve_noalloc(pf_batch *b, int n_scen, const int *
         BatchTopo tp = nb.tp;
         void *args[] = {&tp, &J};
         BHIP(hipLaunchKernel((const void *)batch_kernel(mixed, nb.mode, plan[i].block), dim3(plan[i].grid),
-                             dim3(plan[i].block), args, nb.mode == 0 ? 0 : (size_t)nb.shm, s));
+                             dim3(plan[i].block), args, (size_t)b->shm_bytes(nb, nb.mode, plan[i].block), s));
     }
     if (!stream) {
         BHIP(hipStreamSynchronize(s));

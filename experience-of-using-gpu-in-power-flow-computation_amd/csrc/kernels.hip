@@ -580,7 +580,7 @@ __global__ void __launch_bounds__(1024) k_fwd_tail(DevSym Y, const T *blk, doubl
         pL = nL;
     }
     __shared__ double s_r[2 * kChainMax];
-    if (Y.ch_m > 0) chain_solve<T, 16>(Y, blk, x, s_r);
+    if (Y.ch_m > 0) chain_solve<T, 16>(Y, blk, x, s_r, Y.rs_ptr);
 }
 
 template <typename T>
@@ -764,7 +764,7 @@ __global__ void __launch_bounds__(1024) k_fwd_tail_lds(DevSym Y, DevTail D, cons
     }
     __syncthreads();
     __shared__ double s_r[2 * kChainMax];
-    if (Y.ch_m > 0) chain_solve<T, 16>(Y, blk, x, s_r);
+    if (Y.ch_m > 0) chain_solve<T, 16>(Y, blk, x, s_r, Y.rs_ptr);
 }
 
 // levels [lv0, lv1) of the tail, backward, after k_tail_bwd_ext

@@ -876,17 +876,17 @@ __device__ __forceinline__ void chain_factor_mem(const DevSym &Y, T *blk, int *b
 
 // Chain part of a solve, after the forward sweep over the levels before the
 // chain: x_C <- S^-1 (x_C - L_CN x_N), where x_C still holds the right-hand
-// side (s_r: 2 ch_m doubles of LDS).  The backward sweep then starts below
+// side (s_r: 2 ch_m doubles of LDS; rs: the row pointers).  The backward sweep then starts below
 // the chain.  Two barriers.
-template <typename T, int G>
-__device__ __forceinline__ void chain_solve(const DevSym &Y, const T *blk, double *x, double *s_r) {
+template <typename T, int G, typename PTR>
+__device__ __forceinline__ void chain_solve(const DevSym &Y, const T *blk, double *x, double *s_r, const PTR rs) {
     const int m = Y.ch_m, c0 = Y.ch_c0;
     const int LR0 = Y.n + 2 * Y.nnzL, SB = Y.n + 3 * Y.nnzL;
     const int tid = (int)threadIdx.x, grp = tid / G, lane = tid % G, ng = (int)blockDim.x / G;
     for (int a = grp; a < m; a += ng) {
         const int c = c0 + a;
         double a0 = 0, a1 = 0;
-        for (int q = Y.rs_ptr[c] + lane; q < Y.rs_ptr[c + 1]; q += G) {
+        for (int q = rs[c] + lane, qe = rs[c + 1]; q < qe; q += G) {
             const int k = Y.rs_k[q];
             if (k >= c0) break;                 // row entries ascend in k
             const B4<T> L = load_b4(blk, LR0 + q);

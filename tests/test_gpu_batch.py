@@ -389,3 +389,65 @@ def test_batch_odd_size_network(pf, oracle, synth, precision):
                 if precision == "fp64":
                     assert it[s] == r["iterations"], (mode, s)
     assert 2 in ran
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("copies,n", [(2, 257), (3, 600), (5, 300), (5, 513)])
+def test_batch_several_workgroups_a_cu(pf, oracle, synth, tmp_path, precision, copies, n):
+    """More scenarios than CUs of a network beyond LDS: several narrow workgroups share a CU, with less
+    LDS each.  The bits are those of one wide workgroup per CU; the answers (the first and last
+    scenario) are the oracle's."""
+    path = str(tmp_path / "c.cdfx")
+    synth.write_cdf(synth.multi_copy(copies, 118000, 2 * copies, copies), path, wide=True)
+    net, oc = pf.Network(path), oracle.Case(path)
+    P, Q, L = _scenarios(synth, net, n, 3800000)
+    b = pf.Batch([net], pf.options(tolerancia=1e-8, no_max_iter=30, lim_inj_reat=1,
+                                   precision=pf.MIXED if precision == "mixed" else pf.FP64))
+    b.set_scenarios(np.zeros(n, np.int32), P.ravel(), Q.ravel(), L.ravel())
+    shape = b.shape(0)
+    _say(copies, n, precision, shape)
+    assert shape["mode"] == 1 and shape["block"] < 1024 and shape["grid"] > 256
+    b.solve()
+    got = b.results() + (b.limq()[1],)
+    b.set_shape(0, 1, 1024, 1)
+    b.solve()
+    for x, y in zip(got, b.results() + (b.limq()[1],)):
+        assert np.array_equal(x, y, equal_nan=x.dtype.kind == "f")
+    V, th, it, cv = got[:4]
+    for s, r in zip((0, n - 1), _oracle_solve(oc, P[[0, n - 1]], Q[[0, n - 1]], L[[0, n - 1]])):
+        assert bool(cv[s]) == bool(r["converged"])
+        if cv[s]:
+            k = slice(net.nB * s, net.nB * (s + 1))
+            assert np.abs(V[k] - r["V"]).max() <= 1e-6 and np.abs(th[k] - r["theta"]).max() <= 1e-6
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_batch_long_row_pointers(pf, synth, tmp_path, precision):
+    """A complete graph of 384 buses has 73,153 entries in L, past 16 bits: the narrow workgroups' sweeps
+    read the row and column pointers where they are in memory.  Same bits at every size; the single
+    solver's answer within 1e-9."""
+    rng = np.random.default_rng(5)
+    nb = 384
+    buses = [synth.Bus(i + 1, 3 if i == 0 else 0, pload=round(float(rng.uniform(0, 2)), 1) * (i > 0),
+                       qload=round(float(rng.uniform(0, 0.5)), 1) * (i > 0)) for i in range(nb)]
+    branches = [synth.Branch(i + 1, j + 1, 1.0, round(float(rng.uniform(5, 9)), 3))
+                for i in range(nb) for j in range(i + 1, nb)]
+    path = str(tmp_path / "dense.cdf")
+    synth.write_cdf(synth.Case(buses, branches), path)
+    net = pf.Network(path)
+    opts = pf.options(tolerancia=1e-8, no_max_iter=10, precision=pf.MIXED if precision == "mixed" else pf.FP64)
+    b = pf.Batch([net], opts)
+    b.set_scenarios(np.zeros(2, np.int32), *[np.tile(a, 2) for a in (net.Pg - net.Pload, net.Qg - net.Qload, net.Qload)])
+    outs = []
+    for block in (256, 512, 1024):
+        b.set_shape(0, 1, block)
+        b.solve()
+        outs.append(b.results())
+    assert outs[0][3].all()
+    for o in outs[1:]:
+        for x, y in zip(outs[0], o):
+            assert np.array_equal(x, y)
+    s = pf.Solver(net, opts)
+    s.solve(check=True)
+    V, th, _ = s.state()
+    assert np.abs(outs[0][0][:nb] - V).max() <= 1e-9 and np.abs(outs[0][1][:nb] - th).max() <= 1e-9
