@@ -433,26 +433,23 @@ class Batch:
         return {"mode": m.value, "block": b.value, "grid": g.value, "lds_bytes": lds.value}
 
     def results(self):
-        V = np.zeros(self.total)
-        th = np.zeros(self.total)
-        it = np.zeros(self.n_scen, np.int32)
-        cv = np.zeros(self.n_scen, np.int32)
-        mm = np.zeros(self.n_scen)
+        V = np.empty(self.total)
+        th = np.empty(self.total)
+        it = np.empty(self.n_scen, np.int32)
+        cv = np.empty(self.n_scen, np.int32)
+        mm = np.empty(self.n_scen)
         _chk(lib().pf_batch_get(self.h, _p(V), _p(th), _p(it), _p(cv), _p(mm)), "pf_batch_get")
         return V, th, it, cv.astype(bool), mm
 
     def limq(self):
         """Final PV->PQ state per scenario: (list of bool arrays [nPV of the
         scenario's network], flips per scenario)."""
-        npv = [self.nets[i].nPV for i in self.net_of]
-        lq = np.zeros(max(1, sum(npv)), np.uint8)
-        fl = np.zeros(self.n_scen, np.int32)
+        end = np.cumsum(np.array([n.nPV for n in self.nets])[self.net_of])
+        lq = np.empty(max(1, int(end[-1])), np.uint8)
+        fl = np.empty(self.n_scen, np.int32)
         _chk(lib().pf_batch_get_limq(self.h, _p(lq), _p(fl)), "pf_batch_get_limq")
-        out, o = [], 0
-        for k in npv:
-            out.append(lq[o:o + k].astype(bool))
-            o += k
-        return out, fl
+        lq, end = lq.astype(bool), end.tolist()
+        return [lq[a:b] for a, b in zip([0] + end, end)], fl
 
 
 class WarmStart:

@@ -31,6 +31,7 @@
 #include "kernels_decl.hpp"
 #include "kernels_impl.hpp"
 #include "pf_internal.hpp"
+#include "transfer.hpp"
 
 using namespace pf;
 
@@ -1331,6 +1332,7 @@ struct pf_batch {
     long long *d_off = nullptr, *d_pvoff = nullptr;
     unsigned char *d_lq = nullptr;
     int cus = 0;
+    PinnedSlots slots;
 
     template <typename T>
     pf_status alloc(T **p, size_t n) {
@@ -2020,22 +2022,26 @@ pf_status pf_batch_get(pf_batch *b, double *V, double *theta, int *iterations, i
                        double *max_mismatch) {
     if (!b || !b->n_scen) return PF_INVALID_ARG;
     BHIP(hipSetDevice(b->device));
-    BHIP(hipStreamSynchronize(b->st[0]));
-    if (V) BHIP(hipMemcpy(V, b->d_V, sizeof(double) * b->total, hipMemcpyDeviceToHost));
-    if (theta) BHIP(hipMemcpy(theta, b->d_T, sizeof(double) * b->total, hipMemcpyDeviceToHost));
-    if (iterations) BHIP(hipMemcpy(iterations, b->d_it, sizeof(int) * b->n_scen, hipMemcpyDeviceToHost));
-    if (converged) BHIP(hipMemcpy(converged, b->d_cv, sizeof(int) * b->n_scen, hipMemcpyDeviceToHost));
-    if (max_mismatch) BHIP(hipMemcpy(max_mismatch, b->d_mm, sizeof(double) * b->n_scen, hipMemcpyDeviceToHost));
+    const size_t total = (size_t)b->total, n = (size_t)b->n_scen;
+    CopyPiece out[5];
+    int k = 0;
+    if (V) out[k++] = {V, b->d_V, sizeof(double) * total};
+    if (theta) out[k++] = {theta, b->d_T, sizeof(double) * total};
+    if (iterations) out[k++] = {iterations, b->d_it, sizeof(int) * n};
+    if (converged) out[k++] = {converged, b->d_cv, sizeof(int) * n};
+    if (max_mismatch) out[k++] = {max_mismatch, b->d_mm, sizeof(double) * n};
+    BHIP(b->slots.fetch(out, k, b->st[0]));
     return PF_OK;
 }
 
 pf_status pf_batch_get_limq(pf_batch *b, unsigned char *limQ, int *flips) {
     if (!b || !b->n_scen) return PF_INVALID_ARG;
     BHIP(hipSetDevice(b->device));
-    BHIP(hipStreamSynchronize(b->st[0]));
-    if (limQ && b->total_pv > 0)
-        BHIP(hipMemcpy(limQ, b->d_lq, (size_t)b->total_pv, hipMemcpyDeviceToHost));
-    if (flips) BHIP(hipMemcpy(flips, b->d_fl, sizeof(int) * b->n_scen, hipMemcpyDeviceToHost));
+    CopyPiece out[2];
+    int k = 0;
+    if (limQ) out[k++] = {limQ, b->d_lq, (size_t)b->total_pv};
+    if (flips) out[k++] = {flips, b->d_fl, sizeof(int) * (size_t)b->n_scen};
+    BHIP(b->slots.fetch(out, k, b->st[0]));
     return PF_OK;
 }
 

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "pf_internal.hpp"
+#include "transfer.hpp"
 
 typedef __bf16 bf16;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -291,6 +292,7 @@ struct pf_warmstart {
     int Bcap = 0;
     int staged = 0;   // rows of features on the device for pf_warmstart_predict_into
     hipStream_t stream = nullptr;
+    pf::PinnedSlots slots;
     std::vector<void *> allocs, ws_allocs;
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
     bf16 *pb = nullptr;        // the parameters in bf16, laid out as p
@@ -560,7 +562,8 @@ pf_status pf_warmstart_set_norm(pf_warmstart *w, const float *x_mean, const floa
 pf_status pf_warmstart_get_params(pf_warmstart *w, float *out) {
     if (!w || !out) return PF_INVALID_ARG;
     MHIP(hipSetDevice(w->device));
-    MHIP(hipMemcpy(out, w->p, sizeof(float) * w->n_params, hipMemcpyDeviceToHost));
+    const pf::CopyPiece all{out, w->p, sizeof(float) * w->n_params};
+    MHIP(w->slots.fetch(&all, 1, w->stream));
     return PF_OK;
 }
 
@@ -618,8 +621,9 @@ pf_status pf_warmstart_fit(pf_warmstart *w, const float *X, const float *Y, int 
             st = PF_DEVICE_ERROR;
         }
     };
-    ok(hipMemcpy(dX, X, sizeof(float) * (size_t)n * w->n_in, hipMemcpyHostToDevice));
-    ok(hipMemcpy(dY, Y, sizeof(float) * (size_t)n * w->n_out, hipMemcpyHostToDevice));
+    const pf::CopyPiece rows[2] = {{(void *)X, dX, sizeof(float) * (size_t)n * w->n_in},
+                                   {(void *)Y, dY, sizeof(float) * (size_t)n * w->n_out}};
+    ok(w->slots.send(rows, 2, w->stream));
     std::vector<int> perm(n);
     for (int i = 0; i < n; i++) perm[i] = i;
     unsigned long long s = seed;

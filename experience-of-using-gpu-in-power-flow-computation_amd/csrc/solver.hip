@@ -82,7 +82,11 @@ struct pf_solver {
     double *dense = nullptr;
     int *dense_chg = nullptr;   // the dense panel's row swaps
     Ctl *ctl = nullptr;
-    Ctl *ctl_host = nullptr;      // pinned, 2 slots
+    Ctl *ctl_host = nullptr;      // pinned, 2 slots, then the state's copy
+    // what a reset sets and a caller reads, in one block of device memory (V,
+    // theta, QliqLim, isq, limQ) with a pinned copy: one transfer either way
+    char *state_dev = nullptr, *state_host = nullptr;
+    size_t state_bytes = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -114,10 +118,36 @@ struct pf_solver {
         *p = (T *)q;
         return PF_OK;
     }
+    // The plan's small arrays are packed on the host and copied at once by
+    // flush_uploads, which sets their pointers: an allocation and a copy each
+    // took some 15 us, 70 of them half the 2.3 ms of a 118-bus case from file
+    // to report.  From 64 KB on the packing costs as much.
+    struct Upload {
+        void **p;
+        size_t off;
+    };
+    std::vector<Upload> uploads;
+    std::vector<char> packed;
     template <typename T>
     pf_status upload(T **p, const std::vector<T> &v) {
-        PFCHK(alloc(p, v.size()));
-        if (!v.empty()) HIPCHK(hipMemcpy(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+        if (sizeof(T) * v.size() >= 65536) {
+            PFCHK(alloc(p, v.size()));
+            HIPCHK(hipMemcpy(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+            return PF_OK;
+        }
+        uploads.push_back({(void **)p, packed.size()});
+        const char *b = (const char *)v.data();
+        packed.insert(packed.end(), b, b + sizeof(T) * v.size());
+        packed.resize((packed.size() + 255) / 256 * 256);
+        return PF_OK;
+    }
+    pf_status flush_uploads() {
+        char *d = nullptr;
+        PFCHK(alloc(&d, packed.size()));
+        if (!packed.empty()) HIPCHK(hipMemcpy(d, packed.data(), packed.size(), hipMemcpyHostToDevice));
+        for (const Upload &u : uploads) *u.p = d + u.off;
+        uploads.clear();
+        std::vector<char>().swap(packed);
         return PF_OK;
     }
     template <typename T>
@@ -180,7 +210,10 @@ pf_status pf_solver::build() {
     HIPCHK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     HIPCHK(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
     HIPCHK(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
-    HIPCHK(hipHostMalloc((void **)&ctl_host, 2 * sizeof(Ctl), hipHostMallocDefault));
+    state_bytes = (size_t)net.nB * (3 * sizeof(double) + 1) + net.nPV;
+    const size_t ctl_bytes = (2 * sizeof(Ctl) + 63) / 64 * 64;
+    HIPCHK(hipHostMalloc((void **)&ctl_host, ctl_bytes + state_bytes, hipHostMallocDefault));
+    state_host = (char *)ctl_host + ctl_bytes;
     yp = build_ypattern(net);
     // lu_blocked = 0, the straightforward level schedule: one launch per
     // elimination-tree level, levels narrower than kPlainTailWidth nodes in
@@ -246,8 +279,12 @@ pf_status pf_solver::build() {
     PFCHK(upload((double **)&dn.qmax, net.Qmax));
     PFCHK(upload((double **)&dn.vset, net.Vset));
 
-    PFCHK(alloc(&ds.V, nB));
-    PFCHK(alloc(&ds.th, nB));
+    PFCHK(alloc(&state_dev, state_bytes));
+    ds.V = (double *)state_dev;
+    ds.th = ds.V + nB;
+    ds.QliqLim = ds.th + nB;
+    ds.isq = (unsigned char *)(ds.QliqLim + nB);
+    ds.limQ = ds.isq + nB;
     PFCHK(alloc(&ds.E, nB));
     PFCHK(alloc(&ds.I, nB));
     PFCHK(alloc(&ds.P, nB));
@@ -255,9 +292,6 @@ pf_status pf_solver::build() {
     PFCHK(upload((double **)&ds.Pliq, Pliq));
     PFCHK(upload((double **)&ds.Qliq, Qliq));
     PFCHK(upload((double **)&ds.Qload, Qload));
-    PFCHK(alloc(&ds.QliqLim, nB));
-    PFCHK(alloc(&ds.isq, nB));
-    PFCHK(alloc(&ds.limQ, net.nPV));
     PFCHK(alloc(&ds.g, 2 * (size_t)n));
     PFCHK(alloc(&ds.x, 2 * (size_t)n));
     PFCHK(alloc(&ds.r, 2 * (size_t)n));
@@ -321,6 +355,7 @@ pf_status pf_solver::build() {
 
     // Ybus on the device (once per network), timed like the reference's
     // admitancia phase (CPU/main.cpp:47-56)
+    PFCHK(flush_uploads());
     for (auto &e : tev) HIPCHK(hipEventCreate(&e));
     HIPCHK(hipEventRecord(tev[0], stream));
     k_ybus<<<(yp.nnz + 255) / 256, 256, 0, stream>>>(dn, yp.nnz);
@@ -360,11 +395,16 @@ pf_status pf_solver::set_isq_from_limq(const unsigned char *limQ) {
 // flat start (CPU/estrutura/barra.cpp:20-25 + PV/slack fields) and initLim
 // (CPU/limInjReat.cpp:177-207)
 pf_status pf_solver::reset_state() {
-    PFCHK(put(ds.V, net.V.data(), net.nB));
-    PFCHK(put(ds.th, net.theta.data(), net.nB));
-    PFCHK(put(ds.QliqLim, Qliq.data(), net.nB));
-    PFCHK(set_isq_from_limq(nullptr));
-    return PF_OK;
+    HIPCHK(hipStreamSynchronize(stream));   // an earlier copy may still read state_host
+    const size_t nB = net.nB;
+    double *h = (double *)state_host;
+    std::copy(net.V.begin(), net.V.end(), h);
+    std::copy(net.theta.begin(), net.theta.end(), h + nB);
+    std::copy(Qliq.begin(), Qliq.end(), h + 2 * nB);
+    unsigned char *isq = (unsigned char *)(h + 3 * nB);
+    std::fill(isq, isq + nB + net.nPV, 0);
+    for (int k : net.pq) isq[k] = 1;
+    return put(state_dev, (const char *)state_host, state_bytes);
 }
 
 pf_status pf_solver::reset_ctl() {
@@ -905,9 +945,12 @@ pf_status pf_solver_set_injections(pf_solver *s, const double *Pliq, const doubl
 pf_status pf_solver_get_state(pf_solver *s, double *V, double *theta, unsigned char *limQ) {
     if (!s) return PF_INVALID_ARG;
     HIPCHK(hipSetDevice(s->device));
-    if (V) PFCHK(s->get(V, s->ds.V, s->net.nB));
-    if (theta) PFCHK(s->get(theta, s->ds.th, s->net.nB));
-    if (limQ) PFCHK(s->get(limQ, s->ds.limQ, s->net.nPV));
+    PFCHK(s->get(s->state_host, (const char *)s->state_dev, s->state_bytes));
+    const size_t nB = s->net.nB;
+    const double *h = (const double *)s->state_host;
+    if (V) std::copy(h, h + nB, V);
+    if (theta) std::copy(h + nB, h + 2 * nB, theta);
+    if (limQ) std::memcpy(limQ, (const unsigned char *)(h + 3 * nB) + nB, s->net.nPV);
     return PF_OK;
 }
 
@@ -1000,6 +1043,7 @@ pf_status pf_solver::flows(double *Pdp, double *Qdp, double *Ppd, double *Qpd) {
             h[l] = FlowBranch{f, t, yp.br_ft[l], yp.br_tf[l], phif(f, t), phif(t, f), bshf(f, t), bshf(t, f)};
         }
         PFCHK(upload(&flow_br, h));
+        PFCHK(flush_uploads());
         PFCHK(alloc(&flow_out, 4 * (size_t)nL));
     }
     k_flows<<<(nL + 255) / 256, 256, 0, stream>>>(dn, ds, flow_br, nL, flow_out);

@@ -7,6 +7,7 @@ Tolerances: GEMM |dC| <= 1e-4 max|C| (FP32 vs FP64 accumulation of the same
 bf16 operands); gradients: relative L2 error <= 2e-2 and cosine >= 0.999
 (a bf16 rounding decision can flip where FP32 and FP64 pre-activations
 straddle a rounding boundary)."""
+import ctypes
 import os
 import sys
 
@@ -217,3 +218,33 @@ def test_fit_grows_and_keeps_its_rows(pf):
         w.fit(X[:64], Y[:64], epochs=1, batch=8)
         out.append(w.params())
     assert np.array_equal(out[0], out[1]) and np.all(np.isfinite(out[0]))
+
+
+@pytest.mark.parametrize("n_in,n_out,hidden", [(8, 8, 8), (264, 520, 384), (3000, 2000, 512)])
+def test_params_round_trip(pf, n_in, n_out, hidden):
+    """Parameters come back as they went in: within one pinned slot of 1 MiB, across two, and across more
+    than the four there are (10 MB)."""
+    w = pf.WarmStart(n_in, n_out, hidden, 2, seed=3)
+    p = np.random.default_rng(n_in).standard_normal(w.params().size).astype(np.float32)
+    w.set_params(p)
+    assert np.array_equal(w.params(), p)
+
+
+def test_batch_results_in_parts(pf, synth, cases):
+    """513 scenarios of 944 buses: 3.9 MB an array, all arrays in one call as each in a call of its own."""
+    net = pf.Network(cases.path("c944"))
+    n = 513
+    P, Q, L = (np.tile(a, n) for a in (net.Pg - net.Pload, net.Qg - net.Qload, net.Qload))
+    b = pf.Batch([net], pf.options(tolerancia=1e-8, no_max_iter=1, precision=pf.MIXED))
+    f = np.repeat(np.linspace(0.9, 1.0, n), net.nB)
+    b.set_scenarios(np.zeros(n, np.int32), P * f, Q * f, L * f)
+    b.solve()
+    every = b.results()
+    own = [np.full_like(x, -1, dtype=np.int32 if x.dtype == bool else x.dtype) for x in every]
+    for i, x in enumerate(own):
+        args = [None] * 5
+        args[i] = x.ctypes.data_as(ctypes.c_void_p)
+        assert pf.lib().pf_batch_get(b.h, *args) == pf.PF_OK
+    for x, y in zip(every, own):
+        assert np.array_equal(x, y.astype(x.dtype))
+    assert len(np.unique(every[1].reshape(n, net.nB)[:, 5])) == n     # every scenario has angles of its own
