@@ -68,18 +68,18 @@ __global__ void k_init_E(DevNet N, DevState S) {
 // S_k = E_k conj(sum_m Y_km E_m): LPR lanes per bus row, E staged in LDS for
 // a window of buses around the block's rows (bus numbering keeps most
 // neighbours close), gathered from global memory outside the window.
+// Returns in each row's lane 0 whether it has a row (win: LDS).
+constexpr int kPqWin = 192;
 template <int LPR>
-__global__ void __launch_bounds__(256) k_pq(DevNet N, DevState S, int gate) {
+__device__ __forceinline__ bool pq_row(const DevNet &N, const DevState &S, double2 *win, int &row, double &P, double &Q) {
     constexpr int ROWS = 256 / LPR;
-    constexpr int WIN = 192;
-    __shared__ double2 win[ROWS + 2 * WIN];
-    if (gate && S.ctl->done) return;
+    constexpr int WIN = kPqWin;
     const int r0 = blockIdx.x * ROWS;
     const int r1 = min(N.nB, r0 + ROWS);
     const int lo = max(0, r0 - WIN), hi = min(N.nB, r1 + WIN);
     for (int i = threadIdx.x; i < hi - lo; i += blockDim.x) win[i] = S.E[lo + i];
     __syncthreads();
-    const int row = r0 + (int)threadIdx.x / LPR;
+    row = r0 + (int)threadIdx.x / LPR;
     const int lane = (int)threadIdx.x % LPR;
     double ar = 0.0, ai = 0.0;
     if (row < N.nB) {
@@ -93,15 +93,80 @@ __global__ void __launch_bounds__(256) k_pq(DevNet N, DevState S, int gate) {
     }
     ar = xor_sum<LPR>(ar);
     ai = xor_sum<LPR>(ai);
-    if (row < N.nB && lane == 0) {
-        double2 Ek = win[row - lo];
-        S.I[row] = make_double2(ar, ai);
-        S.P[row] = Ek.x * ar + Ek.y * ai;
-        S.Q[row] = Ek.y * ar - Ek.x * ai;
-    }
+    if (row >= N.nB || lane != 0) return false;
+    double2 Ek = win[row - lo];
+    P = Ek.x * ar + Ek.y * ai;
+    Q = Ek.y * ar - Ek.x * ai;
+    S.I[row] = make_double2(ar, ai);
+    S.P[row] = P;
+    S.Q[row] = Q;
+    return true;
+}
+
+template <int LPR>
+__global__ void __launch_bounds__(256) k_pq(DevNet N, DevState S, int gate) {
+    __shared__ double2 win[256 / LPR + 2 * kPqWin];
+    if (gate && S.ctl->done) return;
+    int row;
+    double P, Q;
+    pq_row<LPR>(N, S, win, row, P, Q);
 }
 
 // ---------------------------------------------------------------- limits
+// The rules at PV bus b, the i-th, with power Q: chkLimQ (do_chk) on one that
+// is not limited, undo_chkLimQ on one that is.  Returns the flips, 0 or 1.
+__device__ __forceinline__ int limit_bus(const DevNet &N, const DevState &S, int i, int b, double Q, bool do_chk) {
+    const double qload = S.Qload[b];
+    const double qmin = N.qmin[i], qmax = N.qmax[i];
+    unsigned char lq = S.limQ[i];
+    double qll = S.QliqLim[b];
+    int flips = 0;
+    if (!lq) {
+        if (do_chk) {
+            double qg = Q + qload;
+            if (qg < qmin - kFolga) {
+                qll = qmin - qload;
+                lq = 1;
+                flips++;
+            } else if (qg > qmax + kFolga) {
+                qll = qmax - qload;
+                lq = 1;
+                flips++;
+            }
+        }
+    } else {
+        if (qll == qmax - qload) {
+            if (S.V[b] > N.vset[i] + kFolga) {
+                lq = 0;
+                qll = S.Qliq[b];
+                flips++;
+            }
+        } else {
+            if (S.V[b] < N.vset[i] - kFolga) {
+                lq = 0;
+                qll = S.Qliq[b];
+                flips++;
+            }
+        }
+    }
+    S.limQ[i] = lq;
+    S.QliqLim[b] = qll;
+    S.isq[b] = lq;
+    return flips;
+}
+
+// all PV buses, one workgroup (s_flips: 0 in LDS before, past a barrier)
+__device__ __forceinline__ void limit_buses(const DevNet &N, const DevState &S, bool do_chk, int *s_flips) {
+    int flips = 0;
+    for (int i = threadIdx.x; i < N.nPV; i += blockDim.x) {
+        const int b = N.pv_bus[i];
+        flips += limit_bus(N, S, i, b, S.Q[b], do_chk);
+    }
+    if (flips) atomicAdd(s_flips, flips);
+    __syncthreads();
+    if (threadIdx.x == 0 && *s_flips) atomicAdd(&S.ctl->flips, *s_flips);
+}
+
 // One workgroup.  mode 0: start of a pass (reference trigger at iteration
 // >= 1: chkLimQ when max|previous dx| < 0.1, else undo_chkLimQ if any bus is
 // limited, CPU/newtonRaphson.cpp:202-211); mode 1: switch taken at
@@ -121,69 +186,64 @@ __global__ void __launch_bounds__(1024) k_limits(DevNet N, DevState S, int mode,
     }
     any = __syncthreads_or(any);
     if (!do_chk && !any) return;
-    int flips = 0;
-    for (int i = threadIdx.x; i < N.nPV; i += blockDim.x) {
-        const int b = N.pv_bus[i];
-        const double qload = S.Qload[b];
-        const double qmin = N.qmin[i], qmax = N.qmax[i];
-        unsigned char lq = S.limQ[i];
-        double qll = S.QliqLim[b];
-        if (!lq) {
-            if (do_chk) {
-                double qg = S.Q[b] + qload;
-                if (qg < qmin - kFolga) {
-                    qll = qmin - qload;
-                    lq = 1;
-                    flips++;
-                } else if (qg > qmax + kFolga) {
-                    qll = qmax - qload;
-                    lq = 1;
-                    flips++;
-                }
-            }
-        } else {
-            if (qll == qmax - qload) {
-                if (S.V[b] > N.vset[i] + kFolga) {
-                    lq = 0;
-                    qll = S.Qliq[b];
-                    flips++;
-                }
-            } else {
-                if (S.V[b] < N.vset[i] - kFolga) {
-                    lq = 0;
-                    qll = S.Qliq[b];
-                    flips++;
-                }
-            }
-        }
-        S.limQ[i] = lq;
-        S.QliqLim[b] = qll;
-        S.isq[b] = lq;
-    }
-    if (flips) atomicAdd(&s_flips, flips);
-    __syncthreads();
-    if (threadIdx.x == 0 && s_flips) atomicAdd(&ctl->flips, s_flips);
+    limit_buses(N, S, do_chk, &s_flips);
 }
 
 // --------------------------------------------------------------- mismatch
+// bus k, not the slack: g (and x, the step's right-hand side), the largest of
+// it and whether its Q is outside its limits
+__device__ __forceinline__ void mismatch_bus(const DevNet &N, const DevState &S, int k, double P, double Q, bool to_x,
+                                             double &m, unsigned &bad) {
+    int j = N.node_of_bus[k];
+    double gp = S.Pliq[k] - P;
+    double gq = S.isq[k] ? S.QliqLim[k] - Q : 0.0;
+    S.g[2 * j] = gp;
+    S.g[2 * j + 1] = gq;
+    if (to_x) {
+        S.x[2 * j] = gp;
+        S.x[2 * j + 1] = gq;
+    }
+    m = dmax_nan(fabs(gp), fabs(gq));
+    int i = N.pv_of_bus[k];
+    if (i >= 0) {
+        double qg = Q + S.Qload[k];
+        bad = (qg < N.qmin[i] - kFolga) || (qg > N.qmax[i] + kFolga);
+    }
+}
+
+// The first half of a pass, a bus row at a time: P and Q, the limits' rules
+// at iteration >= 1 (k_limits, mode 0: what a bus does depends on its own
+// numbers and on max|previous dx| alone), g.  In place of three launches and a
+// copy of g to x, which cost what an empty launch costs at these sizes (4 to 8
+// us each).
+template <int LPR>
+__global__ void __launch_bounds__(256) k_head(DevNet N, DevState S, int lim) {
+    __shared__ double2 win[256 / LPR + 2 * kPqWin];
+    Ctl *ctl = S.ctl;
+    if (ctl->done) return;
+    int k;
+    double P, Q, m = 0.0;
+    unsigned bad = 0;
+    if (pq_row<LPR>(N, S, win, k, P, Q) && k != N.slack) {
+        const int i = N.pv_of_bus[k];
+        if (lim && i >= 0 && ctl->it >= 1 && limit_bus(N, S, i, k, Q, u64_as_double(ctl->maxDx_bits) < 0.1))
+            atomicAdd(&ctl->flips, 1);
+        mismatch_bus(N, S, k, P, Q, true, m, bad);
+    }
+    m = wave_max(m);
+    bad = __any(bad);
+    if ((threadIdx.x & 63) == 0) {
+        atomicMax(&ctl->maxG_bits, double_as_u64(m));
+        if (bad) atomicOr(&ctl->simple_bad, 1u);
+    }
+}
+
 __global__ void __launch_bounds__(256) k_mismatch(DevNet N, DevState S, int gate) {
     if (gate && S.ctl->done) return;
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     double m = 0.0;
     unsigned bad = 0;
-    if (k < N.nB && k != N.slack) {
-        int j = N.node_of_bus[k];
-        double gp = S.Pliq[k] - S.P[k];
-        double gq = S.isq[k] ? S.QliqLim[k] - S.Q[k] : 0.0;
-        S.g[2 * j] = gp;
-        S.g[2 * j + 1] = gq;
-        m = dmax_nan(fabs(gp), fabs(gq));
-        int i = N.pv_of_bus[k];
-        if (i >= 0) {
-            double qg = S.Q[k] + S.Qload[k];
-            bad = (qg < N.qmin[i] - kFolga) || (qg > N.qmax[i] + kFolga);
-        }
-    }
+    if (k < N.nB && k != N.slack) mismatch_bus(N, S, k, S.P[k], S.Q[k], false, m, bad);
     m = wave_max(m);
     bad = __any(bad);
     if ((threadIdx.x & 63) == 0) {
@@ -194,9 +254,7 @@ __global__ void __launch_bounds__(256) k_mismatch(DevNet N, DevState S, int gate
 
 // Decision of a pass (CPU/newtonRaphson.cpp:247-264): converged, switch at
 // convergence (zero step, as the reference's step there is O(tol)), or step.
-__global__ void k_control(DevState S, int lim) {
-    if (threadIdx.x != 0) return;
-    Ctl *c = S.ctl;
+__device__ __forceinline__ void control(Ctl *c, int lim) {
     if (c->done) return;
     double maxG = u64_as_double(c->maxG_bits);
     c->maxG = maxG;
@@ -218,6 +276,22 @@ __global__ void k_control(DevState S, int lim) {
     c->maxG_bits = 0;
     c->simple_bad = 0;
     c->maxDx_bits = 0;
+}
+
+__global__ void k_control(DevState S, int lim) {
+    if (threadIdx.x == 0) control(S.ctl, lim);
+}
+
+// with the switch at convergence behind it (k_limits, mode 1), one workgroup
+__global__ void __launch_bounds__(1024) k_decide(DevNet N, DevState S, int lim) {
+    __shared__ int s_post, s_flips;
+    if (threadIdx.x == 0) {
+        control(S.ctl, lim);
+        s_post = S.ctl->post;
+        s_flips = 0;
+    }
+    __syncthreads();
+    if (s_post) limit_buses(N, S, true, &s_flips);
 }
 
 // ----------------------------------------------------------- Jacobian fill
@@ -1023,17 +1097,17 @@ __global__ void __launch_bounds__(256) k_residual(DevNet N, DevState S, int gate
 }
 
 // ----------------------------------------------------------------- update
-__global__ void __launch_bounds__(256) k_update(DevNet N, DevState S, int gate) {
+__global__ void __launch_bounds__(256) k_update(DevNet N, DevState S, int add_r, int gate) {
     if (gate && !S.ctl->step) return;
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     double m = 0.0;
     if (k < N.nB && k != N.slack) {
         const int j = N.node_of_bus[k];
-        const double dth = S.x[2 * j];
+        const double dth = add_r ? S.x[2 * j] + S.r[2 * j] : S.x[2 * j];
         double v = S.V[k], th = S.th[k] + dth;
         m = fabs(dth);
         if (S.isq[k]) {
-            const double dv = S.x[2 * j + 1];
+            const double dv = add_r ? S.x[2 * j + 1] + S.r[2 * j + 1] : S.x[2 * j + 1];
             v += dv;
             m = dmax_nan(m, fabs(dv));
         }
@@ -1074,6 +1148,7 @@ __global__ void k_dense_scatter(DevSym Y, const double *blk, double *A, int ld, 
 }
 
 // explicit instantiations
+template __global__ void k_head<4>(DevNet, DevState, int);
 template __global__ void k_pq<4>(DevNet, DevState, int);
 template __global__ void k_residual<4>(DevNet, DevState, int);
 template __global__ void k_jfill<double>(DevNet, DevState, DevSym, double *, int);

@@ -3,11 +3,13 @@
 // the stage entry points.
 //
 // One NR pass (CPU/newtonRaphson.cpp:180-305, GPU/newtonRaphson.cuh:283-560):
-//   k_pq -> [k_limits: trigger] -> k_mismatch -> k_control -> [k_limits: switch
-//   at convergence] -> step: k_jfill -> factor -> solves (-> refinement) -> k_update
-// Every kernel after k_control is gated on the device flag ctl->step, and
-// every kernel before it on ctl->done, so a captured pass can be replayed
-// until the device says it converged; the host polls one small struct.
+//   k_head (P and Q, limits' trigger, mismatch) -> k_decide (and the switch at
+//   convergence) -> step: k_jfill -> factor -> solves (-> refinement) -> k_update
+// (k_pq, k_limits, k_mismatch and k_control are these one by one, for stage
+// timing and the stage entry points.)  Every kernel after k_decide is gated
+// on the device flag ctl->step, and every kernel before it on ctl->done, so a
+// captured pass can be replayed until the device says it converged; the host
+// polls one small struct.
 
 #include <hip/hip_runtime.h>
 
@@ -187,8 +189,8 @@ struct pf_solver {
     pf_status flows(double *Pdp, double *Qdp, double *Ppd, double *Qpd);
     pf_status set_isq_from_limq(const unsigned char *limQ);
     pf_status reset_ctl();
-    pf_status enqueue_head(int gate);
-    pf_status enqueue_factor_solve(int gate);
+    pf_status enqueue_head();
+    pf_status enqueue_factor_solve(int gate, bool sum);
     pf_status setup_tail_sweeps();
     pf_status setup_flat_tail();
     pf_status upload_flat(const FlatTail &ft, DevFlat &F);
@@ -419,15 +421,22 @@ pf_status pf_solver::reset_ctl() {
 
 // ------------------------------------------------------- launch sequences
 
-pf_status pf_solver::enqueue_head(int gate) {
+// P and Q, limits, g and the decision (stage timing keeps P and Q by itself)
+pf_status pf_solver::enqueue_head() {
     const int nB = net.nB;
     mark(0);
-    k_pq<4><<<(nB + 63) / 64, 256, 0, stream>>>(dn, ds, gate);
-    mark(1);
-    if (lim()) k_limits<<<1, 1024, 0, stream>>>(dn, ds, 0, 1);
-    k_mismatch<<<(nB + 255) / 256, 256, 0, stream>>>(dn, ds, gate);
-    k_control<<<1, 64, 0, stream>>>(ds, lim());
-    if (lim()) k_limits<<<1, 1024, 0, stream>>>(dn, ds, 1, 1);
+    if (!timing) {
+        k_head<4><<<(nB + 63) / 64, 256, 0, stream>>>(dn, ds, lim());
+        k_decide<<<1, lim() ? 1024 : 64, 0, stream>>>(dn, ds, lim());
+    } else {
+        k_pq<4><<<(nB + 63) / 64, 256, 0, stream>>>(dn, ds, 1);
+        mark(1);
+        if (lim()) k_limits<<<1, 1024, 0, stream>>>(dn, ds, 0, 1);
+        k_mismatch<<<(nB + 255) / 256, 256, 0, stream>>>(dn, ds, 1);
+        k_control<<<1, 64, 0, stream>>>(ds, lim());
+        if (lim()) k_limits<<<1, 1024, 0, stream>>>(dn, ds, 1, 1);
+        k_copy<<<(2 * sym.n + 255) / 256, 256, 0, stream>>>(ds.x, ds.g, 2 * sym.n, ctl, 1);
+    }
     HIPCHK(hipGetLastError());
     return PF_OK;
 }
@@ -658,8 +667,9 @@ pf_status pf_solver::enqueue_solve(const T *blk, double *v, int gate) {
     return PF_OK;
 }
 
-// factor at the current state and solve J x = g (x, in node order)
-pf_status pf_solver::enqueue_factor_solve(int gate) {
+// factor at the current state and solve J x = g from x = g (x, in node order;
+// sum: with the last correction added to it, else that one is left in r)
+pf_status pf_solver::enqueue_factor_solve(int gate, bool sum) {
     const int m = 2 * sym.n;
     if (path() == PF_DENSO) {
         PFCHK(ensure_dense());
@@ -669,20 +679,18 @@ pf_status pf_solver::enqueue_factor_solve(int gate) {
         size_t mm = (size_t)m * m;
         k_fill<<<(unsigned)((mm + 255) / 256), 256, 0, stream>>>(dense, mm, 0.0);
         k_dense_scatter<<<(sym.nslot() + 255) / 256, 256, 0, stream>>>(dy, blk64, dense, m, ctl, gate);
-        k_copy<<<(m + 255) / 256, 256, 0, stream>>>(ds.x, ds.g, m, ctl, gate);
         launch_dense_solve(dense, ds.x, m, dense_chg, ctl, gate, stream);
     } else if (mixed()) {
         PFCHK(enqueue_lu(blk32, gate));
-        k_copy<<<(m + 255) / 256, 256, 0, stream>>>(ds.x, ds.g, m, ctl, gate);
         PFCHK(enqueue_solve((const float *)blk32, ds.x, gate));
         for (int r = 0; r < opt.refine_steps; r++) {
             k_residual<4><<<(net.nB + 63) / 64, 256, 0, stream>>>(dn, ds, gate);
             PFCHK(enqueue_solve((const float *)blk32, ds.r, gate));
-            k_axpy<<<(m + 255) / 256, 256, 0, stream>>>(ds.x, ds.r, m, ctl, gate);
+            if (sum || r + 1 < opt.refine_steps)
+                k_axpy<<<(m + 255) / 256, 256, 0, stream>>>(ds.x, ds.r, m, ctl, gate);
         }
     } else {
         PFCHK(enqueue_lu(blk64, gate));
-        k_copy<<<(m + 255) / 256, 256, 0, stream>>>(ds.x, ds.g, m, ctl, gate);
         PFCHK(enqueue_solve((const double *)blk64, ds.x, gate));
     }
     HIPCHK(hipGetLastError());
@@ -690,9 +698,9 @@ pf_status pf_solver::enqueue_factor_solve(int gate) {
 }
 
 pf_status pf_solver::enqueue_step(int gate) {
-    PFCHK(enqueue_factor_solve(gate));
+    PFCHK(enqueue_factor_solve(gate, false));
     mark(4);
-    k_update<<<(net.nB + 255) / 256, 256, 0, stream>>>(dn, ds, gate);
+    k_update<<<(net.nB + 255) / 256, 256, 0, stream>>>(dn, ds, mixed() && opt.refine_steps > 0, gate);
     mark(5);
     HIPCHK(hipGetLastError());
     return PF_OK;
@@ -722,7 +730,7 @@ pf_status pf_solver::run_hybrid_step() {
     HIPCHK(hipStreamSynchronize(stream));
     hybrid_linear_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - h0).count();
     mark(4);
-    k_update<<<(net.nB + 255) / 256, 256, 0, stream>>>(dn, ds, 1);
+    k_update<<<(net.nB + 255) / 256, 256, 0, stream>>>(dn, ds, 0, 1);
     HIPCHK(hipGetLastError());
     mark(5);
     return PF_OK;
@@ -803,7 +811,7 @@ pf_status pf_solver::solve(pf_result *res) {
     if (opt.use_graph && path() == PF_ESPARSO && !timing && !trace_cb) {
         if (!gexec) {
             HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-            pf_status st = enqueue_head(1);
+            pf_status st = enqueue_head();
             if (st == PF_OK) st = enqueue_step(1);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(stream, &g);
@@ -839,7 +847,7 @@ pf_status pf_solver::solve(pf_result *res) {
         }
         double pass_ms[4];
         for (int it = 0; it < maxit; it++) {
-            PFCHK(enqueue_head(1));
+            PFCHK(enqueue_head());
             if (path() == PF_HIBRIDO_C) {
                 PFCHK(get(&c, ctl, 1));
                 const Ctl head = c;
@@ -1206,7 +1214,8 @@ pf_status pf_stage_lu_solve(pf_solver *s, const double *V, const double *theta,
         xn = gn;
         host_block_solve(s->sym, b.data(), xn.data());
     } else {
-        PFCHK(s->enqueue_factor_solve(1));
+        k_copy<<<(2 * n + 255) / 256, 256, 0, s->stream>>>(s->ds.x, s->ds.g, 2 * n, s->ctl, 1);
+        PFCHK(s->enqueue_factor_solve(1, true));
         PFCHK(s->get(xn.data(), s->ds.x, xn.size()));
         PFCHK(s->get(&c, s->ctl, 1));
         if (c.singular) return PF_SINGULAR;

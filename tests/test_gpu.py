@@ -447,3 +447,20 @@ def test_nr_one_workgroup_singular(pf, cases):
         r = s.solve()
         got.append((r["status"], r["iterations"], r["converged"], r["singular"]))
     assert got[0] == got[1] and got[0][3]
+
+
+@pytest.mark.parametrize("precision,refine", [("fp64", 1), ("mixed", 0), ("mixed", 1), ("mixed", 2)])
+def test_nr_head_in_one_launch(pf, cases, precision, refine):
+    """Stage timing runs P/Q, limits, mismatch and decision one by one; without it one launch does the first
+    three and one the decision, and the last correction is added where the state is updated.  Same bits."""
+    net = pf.Network(_path(cases, "c944"))
+    for lim in (0, 1):
+        got = []
+        for timing in (False, True):
+            s = pf.Solver(net, pf.options(tolerancia=1e-6, no_max_iter=40, lim_inj_reat=lim, refine_steps=refine,
+                                          precision=pf.MIXED if precision == "mixed" else pf.FP64))
+            pf.lib().pf_solver_set_timing(s.h, int(timing))
+            r = s.solve()
+            got.append([r[k] for k in ("status", "iterations", "converged", "n_switch_events", "max_mismatch")]
+                       + [x.tobytes() for x in s.state()])
+        assert got[0] == got[1] and got[0][2]
