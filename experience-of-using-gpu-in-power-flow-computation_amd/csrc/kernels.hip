@@ -217,10 +217,10 @@ __device__ __forceinline__ void mismatch_bus(const DevNet &N, const DevState &S,
 // copy of g to x, which cost what an empty launch costs at these sizes (4 to 8
 // us each).
 template <int LPR>
-__global__ void __launch_bounds__(256) k_head(DevNet N, DevState S, int lim) {
+__global__ void __launch_bounds__(256) k_head(DevNet N, DevState S, int lim, int halt) {
     __shared__ double2 win[256 / LPR + 2 * kPqWin];
     Ctl *ctl = S.ctl;
-    if (ctl->done) return;
+    if (ctl->done || (halt && ctl->singular)) return;
     int k;
     double P, Q, m = 0.0;
     unsigned bad = 0;
@@ -283,8 +283,12 @@ __global__ void k_control(DevState S, int lim) {
 }
 
 // with the switch at convergence behind it (k_limits, mode 1), one workgroup
-__global__ void __launch_bounds__(1024) k_decide(DevNet N, DevState S, int lim) {
+__global__ void __launch_bounds__(1024) k_decide(DevNet N, DevState S, int lim, int halt) {
     __shared__ int s_post, s_flips;
+    if (halt && S.ctl->singular) {   // every thread: only the factorisation sets it
+        if (threadIdx.x == 0) S.ctl->step = 0;
+        return;
+    }
     if (threadIdx.x == 0) {
         control(S.ctl, lim);
         s_post = S.ctl->post;
@@ -1148,7 +1152,7 @@ __global__ void k_dense_scatter(DevSym Y, const double *blk, double *A, int ld, 
 }
 
 // explicit instantiations
-template __global__ void k_head<4>(DevNet, DevState, int);
+template __global__ void k_head<4>(DevNet, DevState, int, int);
 template __global__ void k_pq<4>(DevNet, DevState, int);
 template __global__ void k_residual<4>(DevNet, DevState, int);
 template __global__ void k_jfill<double>(DevNet, DevState, DevSym, double *, int);

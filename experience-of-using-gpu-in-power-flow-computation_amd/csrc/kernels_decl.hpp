@@ -11,8 +11,8 @@ template <int LPR> __global__ void k_pq(DevNet N, DevState S, int gate);
 __global__ void k_limits(DevNet N, DevState S, int mode, int lim);
 __global__ void k_mismatch(DevNet N, DevState S, int gate);
 __global__ void k_control(DevState S, int lim);
-template <int LPR> __global__ void k_head(DevNet N, DevState S, int lim);
-__global__ void k_decide(DevNet N, DevState S, int lim);
+template <int LPR> __global__ void k_head(DevNet N, DevState S, int lim, int halt);
+__global__ void k_decide(DevNet N, DevState S, int lim, int halt);
 template <typename T> __global__ void k_jfill(DevNet N, DevState S, DevSym Y, T *blk, int gate);
 template <typename T> __global__ void k_factor_level(DevSym Y, T *blk, Ctl *ctl, int l0, int count, int gate);
 template <typename T> __global__ void k_factor_tail(DevSym Y, T *blk, Ctl *ctl, int lv0, int lv1, int gate);

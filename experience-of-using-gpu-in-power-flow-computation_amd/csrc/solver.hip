@@ -189,7 +189,7 @@ struct pf_solver {
     pf_status flows(double *Pdp, double *Qdp, double *Ppd, double *Qpd);
     pf_status set_isq_from_limq(const unsigned char *limQ);
     pf_status reset_ctl();
-    pf_status enqueue_head();
+    pf_status enqueue_head(int halt);
     pf_status enqueue_factor_solve(int gate, bool sum);
     pf_status setup_tail_sweeps();
     pf_status setup_flat_tail();
@@ -421,13 +421,14 @@ pf_status pf_solver::reset_ctl() {
 
 // ------------------------------------------------------- launch sequences
 
-// P and Q, limits, g and the decision (stage timing keeps P and Q by itself)
-pf_status pf_solver::enqueue_head() {
+// P and Q, limits, g and the decision (stage timing keeps P and Q by itself);
+// halt: nothing after a pass whose pivot failed
+pf_status pf_solver::enqueue_head(int halt) {
     const int nB = net.nB;
     mark(0);
     if (!timing) {
-        k_head<4><<<(nB + 63) / 64, 256, 0, stream>>>(dn, ds, lim());
-        k_decide<<<1, lim() ? 1024 : 64, 0, stream>>>(dn, ds, lim());
+        k_head<4><<<(nB + 63) / 64, 256, 0, stream>>>(dn, ds, lim(), halt);
+        k_decide<<<1, lim() ? 1024 : 64, 0, stream>>>(dn, ds, lim(), halt);
     } else {
         k_pq<4><<<(nB + 63) / 64, 256, 0, stream>>>(dn, ds, 1);
         mark(1);
@@ -808,10 +809,11 @@ pf_status pf_solver::solve(pf_result *res) {
     HIPCHK(hipGetLastError());
     const int maxit = opt.no_max_iter;
     Ctl c{};
-    if (opt.use_graph && path() == PF_ESPARSO && !timing && !trace_cb) {
-        if (!gexec) {
+    if (path() != PF_HIBRIDO_C && !timing && !trace_cb) {
+        const bool replay = opt.use_graph && path() == PF_ESPARSO;
+        if (replay && !gexec) {
             HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-            pf_status st = enqueue_head();
+            pf_status st = enqueue_head(0);
             if (st == PF_OK) st = enqueue_step(1);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(stream, &g);
@@ -820,12 +822,19 @@ pf_status pf_solver::solve(pf_result *res) {
             graph = g;
             HIPCHK(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
         }
-        // pipelined polling: replay i+1 is queued before the host waits on the
-        // copy of the control block that follows replay i
+        // pipelined polling: pass i+1 is queued before the host waits on the
+        // copy of the control block that follows pass i.  (A wait and a copy
+        // between the passes left the GPU idle some 25 us in each: 1,062
+        // buses FP64 without a graph 1,664 -> 1,445 us.)
         int launched = 0, checked = 0;
         while (checked < maxit) {
             while (launched < maxit && launched < checked + 2) {
-                HIPCHK(hipGraphLaunch(gexec, stream));
+                if (replay) {
+                    HIPCHK(hipGraphLaunch(gexec, stream));
+                } else {
+                    PFCHK(enqueue_head(1));
+                    PFCHK(enqueue_step(1));
+                }
                 HIPCHK(hipMemcpyAsync(&ctl_host[launched & 1], ctl, sizeof(Ctl), hipMemcpyDeviceToHost, stream));
                 HIPCHK(hipEventRecord(ev[launched & 1], stream));
                 launched++;
@@ -836,8 +845,7 @@ pf_status pf_solver::solve(pf_result *res) {
             if (c.done || c.singular) break;
         }
         HIPCHK(hipStreamSynchronize(stream));
-        c = ctl_host[(checked - 1) & 1];
-        PFCHK(get(&c, ctl, 1));
+        if (replay) PFCHK(get(&c, ctl, 1));
     } else {
         if (trace_cb) {
             trace_lq.assign(net.nPV, 0);
@@ -847,7 +855,7 @@ pf_status pf_solver::solve(pf_result *res) {
         }
         double pass_ms[4];
         for (int it = 0; it < maxit; it++) {
-            PFCHK(enqueue_head());
+            PFCHK(enqueue_head(0));
             if (path() == PF_HIBRIDO_C) {
                 PFCHK(get(&c, ctl, 1));
                 const Ctl head = c;

@@ -464,3 +464,20 @@ def test_nr_head_in_one_launch(pf, cases, precision, refine):
             got.append([r[k] for k in ("status", "iterations", "converged", "n_switch_events", "max_mismatch")]
                        + [x.tobytes() for x in s.state()])
         assert got[0] == got[1] and got[0][2]
+
+
+@pytest.mark.parametrize("name,precision,metodo", [("c944", "fp64", "ESPARSO"), ("c944", "mixed", "ESPARSO"),
+                                                   ("c118", "fp64", "DENSO")])
+def test_nr_singular_with_a_pass_ahead(pf, cases, name, precision, metodo):
+    """The host queues a pass before it has read the last one's outcome; behind a pass whose pivot failed
+    nothing runs, so outcome and state are those of the solver that waits (stage timing)."""
+    net = pf.Network(_path(cases, name))
+    got = []
+    for timing in (False, True):
+        s = pf.Solver(net, pf.options(tolerancia=1e-8, no_max_iter=10, metodo=getattr(pf, metodo),
+                                      precision=pf.MIXED if precision == "mixed" else pf.FP64))
+        pf.lib().pf_solver_set_timing(s.h, int(timing))
+        s.set_state(np.zeros(net.nB), np.zeros(net.nB))
+        r = s.solve()
+        got.append([r[k] for k in ("status", "iterations", "converged", "singular")] + [x.tobytes() for x in s.state()])
+    assert got[0] == got[1] and got[0][3]
