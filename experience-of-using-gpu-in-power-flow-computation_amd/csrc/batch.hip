@@ -1348,6 +1348,13 @@ struct pf_batch {
         if (!v.empty()) BHIP(hipMemcpy(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
         return PF_OK;
     }
+    PackedUploads plan;   // a network's small arrays, until add_net copies them
+    template <typename T>
+    pf_status plan_array(T **p, const std::vector<T> &v) {
+        if (!PackedUploads::small(v)) return upload(p, v);
+        plan.add(p, v);
+        return PF_OK;
+    }
     ~pf_batch() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
@@ -1405,57 +1412,57 @@ pf_status pf_batch::add_net(const pf_network &src) {
     DevNet &N = b->tp.N;
     DevSym &Y = b->tp.Y;
     N.nB = nB; N.nL = net.nL; N.slack = sl; N.nPV = net.nPV; N.n = n;
-    BCHK(upload((int **)&N.rowptr, yp.rowptr));
-    BCHK(upload((int **)&N.colind, yp.colind));
-    BCHK(upload((int **)&N.coorow, yp.coorow));
-    BCHK(upload((int **)&N.ydiag, yp.diag));
-    BCHK(upload((int **)&N.yc_ptr, yp.contrib_ptr));
-    BCHK(upload((int **)&N.yc, yp.contrib));
-    BCHK(upload((double **)&N.br_r, net.r));
-    BCHK(upload((double **)&N.br_x, net.x));
-    BCHK(upload((double **)&N.br_b, net.bch));
-    BCHK(upload((double **)&N.br_tr, net.tap_re));
-    BCHK(upload((double **)&N.br_ti, net.tap_im));
-    BCHK(upload((double **)&N.gsh, net.gsh));
-    BCHK(upload((double **)&N.bsh, net.bsh));
+    BCHK(plan_array((int **)&N.rowptr, yp.rowptr));
+    BCHK(plan_array((int **)&N.colind, yp.colind));
+    BCHK(plan_array((int **)&N.coorow, yp.coorow));
+    BCHK(plan_array((int **)&N.ydiag, yp.diag));
+    BCHK(plan_array((int **)&N.yc_ptr, yp.contrib_ptr));
+    BCHK(plan_array((int **)&N.yc, yp.contrib));
+    BCHK(plan_array((double **)&N.br_r, net.r));
+    BCHK(plan_array((double **)&N.br_x, net.x));
+    BCHK(plan_array((double **)&N.br_b, net.bch));
+    BCHK(plan_array((double **)&N.br_tr, net.tap_re));
+    BCHK(plan_array((double **)&N.br_ti, net.tap_im));
+    BCHK(plan_array((double **)&N.gsh, net.gsh));
+    BCHK(plan_array((double **)&N.bsh, net.bsh));
     BCHK(alloc(&N.y, yp.nnz));
-    BCHK(upload((int **)&N.node_of_bus, node_of_bus));
+    BCHK(plan_array((int **)&N.node_of_bus, node_of_bus));
     N.bus_of_node = nullptr;
-    BCHK(upload((int **)&N.pv_bus, net.pv));
-    BCHK(upload((int **)&N.pv_of_bus, pv_of_bus));
-    BCHK(upload((double **)&N.qmin, net.Qmin));
-    BCHK(upload((double **)&N.qmax, net.Qmax));
-    BCHK(upload((double **)&N.vset, net.Vset));
+    BCHK(plan_array((int **)&N.pv_bus, net.pv));
+    BCHK(plan_array((int **)&N.pv_of_bus, pv_of_bus));
+    BCHK(plan_array((double **)&N.qmin, net.Qmin));
+    BCHK(plan_array((double **)&N.qmax, net.Qmax));
+    BCHK(plan_array((double **)&N.vset, net.Vset));
     Y.n = n; Y.nnzL = sym.nnzL; Y.nslot = sym.nslot(); Y.nlev = sym.nlev;
     Y.ch_m = sym.ch_m; Y.ch_c0 = sym.ch_c0; Y.nlev_s = sym.nlev_s; Y.di0 = sym.di0();
-    BCHK(upload((int **)&Y.ch_split, sym.ch_split));
-    BCHK(upload((int **)&Y.colptr, sym.colptr));
-    BCHK(upload((int **)&Y.rowind, sym.rowind));
+    BCHK(plan_array((int **)&Y.ch_split, sym.ch_split));
+    BCHK(plan_array((int **)&Y.colptr, sym.colptr));
+    BCHK(plan_array((int **)&Y.rowind, sym.rowind));
     Y.pcol = nullptr;
-    BCHK(upload((int **)&Y.lvl_ptr, sym.lvl_ptr));
-    BCHK(upload((int **)&Y.lvl_nodes, sym.lvl_nodes));
-    BCHK(upload((int **)&Y.fd_ptr, sym.fd_ptr));
-    BCHK(upload((int **)&Y.fc_ptr, sym.fc_ptr));
-    BCHK(upload((int **)&Y.fc_a, sym.fc_a));
-    BCHK(upload((int **)&Y.fc_b, sym.fc_b));
-    BCHK(upload((int **)&Y.rs_ptr, sym.rs_ptr));
-    BCHK(upload((int **)&Y.rs_k, sym.rs_k));
-    BCHK(upload((int **)&Y.rs_p, sym.rs_p));
-    BCHK(upload((int **)&Y.lr_pos, sym.lr_pos));
-    BCHK(upload((int **)&Y.slot_e, sym.slot_e));
-    BCHK(upload((int **)&Y.ld_ptr, sym.ld_ptr));
-    BCHK(upload((int **)&Y.ld_node, sym.ld_node));
-    BCHK(upload((int **)&Y.ld_d, sym.ld_d));
+    BCHK(plan_array((int **)&Y.lvl_ptr, sym.lvl_ptr));
+    BCHK(plan_array((int **)&Y.lvl_nodes, sym.lvl_nodes));
+    BCHK(plan_array((int **)&Y.fd_ptr, sym.fd_ptr));
+    BCHK(plan_array((int **)&Y.fc_ptr, sym.fc_ptr));
+    BCHK(plan_array((int **)&Y.fc_a, sym.fc_a));
+    BCHK(plan_array((int **)&Y.fc_b, sym.fc_b));
+    BCHK(plan_array((int **)&Y.rs_ptr, sym.rs_ptr));
+    BCHK(plan_array((int **)&Y.rs_k, sym.rs_k));
+    BCHK(plan_array((int **)&Y.rs_p, sym.rs_p));
+    BCHK(plan_array((int **)&Y.lr_pos, sym.lr_pos));
+    BCHK(plan_array((int **)&Y.slot_e, sym.slot_e));
+    BCHK(plan_array((int **)&Y.ld_ptr, sym.ld_ptr));
+    BCHK(plan_array((int **)&Y.ld_node, sym.ld_node));
+    BCHK(plan_array((int **)&Y.ld_d, sym.ld_d));
     Y.tail_start = sym.tail_start;
     Y.te0 = sym.ld_ptr[sym.tail_start];
     Y.ck_lvl = Y.ck_q0 = Y.ck_q1 = Y.te_node = Y.te_p = Y.te_ck = nullptr;
     if (opt.lu_blocked && sym.ck_max <= kBatchMaxChunks && !sym.ck_q0.empty()) {
-        BCHK(upload((int **)&Y.ck_lvl, sym.ck_lvl));
-        BCHK(upload((int **)&Y.ck_q0, sym.ck_q0));
-        BCHK(upload((int **)&Y.ck_q1, sym.ck_q1));
-        BCHK(upload((int **)&Y.te_node, sym.te_node));
-        BCHK(upload((int **)&Y.te_p, sym.te_p));
-        BCHK(upload((int **)&Y.te_ck, sym.te_ck));
+        BCHK(plan_array((int **)&Y.ck_lvl, sym.ck_lvl));
+        BCHK(plan_array((int **)&Y.ck_q0, sym.ck_q0));
+        BCHK(plan_array((int **)&Y.ck_q1, sym.ck_q1));
+        BCHK(plan_array((int **)&Y.te_node, sym.te_node));
+        BCHK(plan_array((int **)&Y.te_p, sym.te_p));
+        BCHK(plan_array((int **)&Y.te_ck, sym.te_ck));
     }
     // the factorisation as flat pair lists, its products in the step vectors
     // x and r (4 n doubles, free during the factorisation): from the first
@@ -1481,27 +1488,32 @@ pf_status pf_batch::add_net(const pf_network &src) {
             F.max_pairs = ft.max_pairs;
             F.max_col = ft.max_col;
             F.de_sentinel = ft.de_ptr.back();
-            BCHK(upload((int **)&F.fl_ptr, ft.fl_ptr));
-            BCHK(upload((int **)&F.fl_split, ft.fl_split));
-            BCHK(upload((int **)&F.fl_a, ft.fl_a));
-            BCHK(upload((int **)&F.fl_b, ft.fl_b));
-            BCHK(upload((int **)&F.fl_s, ft.fl_s));
-            BCHK(upload((int **)&F.fl_w, ft.fl_w));
-            BCHK(upload((int **)&F.de_ptr, ft.de_ptr));
-            BCHK(upload((int **)&F.de_node, ft.de_node));
-            BCHK(upload((int **)&F.de_p, ft.de_p));
-            BCHK(upload((int **)&F.de_q0, ft.de_q0));
-            BCHK(upload((int **)&F.de_ext, ft.de_ext));
-            BCHK(upload((int **)&F.de_lo, ft.de_lo));
-            BCHK(upload((int **)&F.de_hi, ft.de_hi));
-            BCHK(upload((int **)&F.de_dlo, ft.de_dlo));
-            BCHK(upload((int **)&F.de_dhi, ft.de_dhi));
-            BCHK(upload((int **)&F.de_lr, ft.de_lr));
-            BCHK(upload((int **)&F.st_g, ft.st_g));
+            BCHK(plan_array((int **)&F.fl_ptr, ft.fl_ptr));
+            BCHK(plan_array((int **)&F.fl_split, ft.fl_split));
+            BCHK(plan_array((int **)&F.fl_a, ft.fl_a));
+            BCHK(plan_array((int **)&F.fl_b, ft.fl_b));
+            BCHK(plan_array((int **)&F.fl_s, ft.fl_s));
+            BCHK(plan_array((int **)&F.fl_w, ft.fl_w));
+            BCHK(plan_array((int **)&F.de_ptr, ft.de_ptr));
+            BCHK(plan_array((int **)&F.de_node, ft.de_node));
+            BCHK(plan_array((int **)&F.de_p, ft.de_p));
+            BCHK(plan_array((int **)&F.de_q0, ft.de_q0));
+            BCHK(plan_array((int **)&F.de_ext, ft.de_ext));
+            BCHK(plan_array((int **)&F.de_lo, ft.de_lo));
+            BCHK(plan_array((int **)&F.de_hi, ft.de_hi));
+            BCHK(plan_array((int **)&F.de_dlo, ft.de_dlo));
+            BCHK(plan_array((int **)&F.de_dhi, ft.de_dhi));
+            BCHK(plan_array((int **)&F.de_lr, ft.de_lr));
+            BCHK(plan_array((int **)&F.st_g, ft.st_g));
         }
     }
-    BCHK(upload((double **)&b->tp.V0flat, net.V));
-    BCHK(upload((double **)&b->tp.th0flat, net.theta));
+    BCHK(plan_array((double **)&b->tp.V0flat, net.V));
+    BCHK(plan_array((double **)&b->tp.th0flat, net.theta));
+    {   // from here on the pointers are set
+        char *d = nullptr;
+        BCHK(alloc(&d, plan.bytes()));
+        BHIP(plan.copy_to(d));
+    }
     b->tp.ck_max = Y.ck_lvl && !b->tp.F.fl_ptr ? sym.ck_max : 0;
     b->tp.nslot = sym.nslot();
     b->tp.nblk = sym.nblk();
@@ -1759,9 +1771,8 @@ pf_status pf_batch_create(const pf_network *const *nets, int n_nets, const pf_op
     BHIP(hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming));
     BHIP(hipEventCreate(&b->t0));
     BHIP(hipEventCreate(&b->t1));
-    hipDeviceProp_t prop;
-    BHIP(hipGetDeviceProperties(&prop, device));
-    b->cus = prop.multiProcessorCount;
+    BHIP(hipDeviceGetAttribute(&b->cus, hipDeviceAttributeMultiprocessorCount, device));
+    BHIP(b->slots.reserve());   // not at the first results
     BCHK(noalloc_setup(device));
     for (int i = 0; i < n_nets; i++) {
         if (!nets[i] || nets[i]->nB < 2 || nets[i]->slack < 0) return PF_INVALID_ARG;

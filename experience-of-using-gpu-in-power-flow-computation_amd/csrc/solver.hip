@@ -25,6 +25,7 @@
 #include "dense.hpp"
 #include "kernels_decl.hpp"
 #include "pf_internal.hpp"
+#include "transfer.hpp"
 
 using namespace pf;
 
@@ -120,36 +121,21 @@ struct pf_solver {
         *p = (T *)q;
         return PF_OK;
     }
-    // The plan's small arrays are packed on the host and copied at once by
-    // flush_uploads, which sets their pointers: an allocation and a copy each
-    // took some 15 us, 70 of them half the 2.3 ms of a 118-bus case from file
-    // to report.  From 64 KB on the packing costs as much.
-    struct Upload {
-        void **p;
-        size_t off;
-    };
-    std::vector<Upload> uploads;
-    std::vector<char> packed;
+    PackedUploads plan;   // small arrays: flush_uploads sets their pointers
     template <typename T>
     pf_status upload(T **p, const std::vector<T> &v) {
-        if (sizeof(T) * v.size() >= 65536) {
-            PFCHK(alloc(p, v.size()));
-            HIPCHK(hipMemcpy(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+        if (PackedUploads::small(v)) {
+            plan.add(p, v);
             return PF_OK;
         }
-        uploads.push_back({(void **)p, packed.size()});
-        const char *b = (const char *)v.data();
-        packed.insert(packed.end(), b, b + sizeof(T) * v.size());
-        packed.resize((packed.size() + 255) / 256 * 256);
+        PFCHK(alloc(p, v.size()));
+        HIPCHK(hipMemcpy(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
         return PF_OK;
     }
     pf_status flush_uploads() {
         char *d = nullptr;
-        PFCHK(alloc(&d, packed.size()));
-        if (!packed.empty()) HIPCHK(hipMemcpy(d, packed.data(), packed.size(), hipMemcpyHostToDevice));
-        for (const Upload &u : uploads) *u.p = d + u.off;
-        uploads.clear();
-        std::vector<char>().swap(packed);
+        PFCHK(alloc(&d, plan.bytes()));
+        HIPCHK(plan.copy_to(d));
         return PF_OK;
     }
     template <typename T>
