@@ -1846,9 +1846,10 @@ pf_status pf_batch_set_scenarios(pf_batch *b, int n_scen, const int *net_of, con
         }
     }
     const size_t tot = (size_t)b->total;
-    BHIP(hipMemcpy(b->d_P, Pliq, sizeof(double) * tot, hipMemcpyHostToDevice));
-    BHIP(hipMemcpy(b->d_Q, Qliq, sizeof(double) * tot, hipMemcpyHostToDevice));
-    BHIP(hipMemcpy(b->d_L, Qload, sizeof(double) * tot, hipMemcpyHostToDevice));
+    const CopyPiece in[3] = {{(void *)Pliq, b->d_P, sizeof(double) * tot},
+                             {(void *)Qliq, b->d_Q, sizeof(double) * tot},
+                             {(void *)Qload, b->d_L, sizeof(double) * tot}};
+    BHIP(b->slots.send(in, 3, b->st[0]));
     const bool had_warm = b->d_V0 != nullptr;
     if (V0) {
         if (!b->warm_V0) {

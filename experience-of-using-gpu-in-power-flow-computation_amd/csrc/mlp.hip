@@ -675,13 +675,14 @@ pf_status pf_warmstart_predict(pf_warmstart *w, const float *X, int B, float *Y)
     w->staged = 0;   // its rows replace the staged ones
     MHIP(hipSetDevice(w->device));
     MCHK(w->ensure(B));
-    MHIP(hipMemcpyAsync(w->X, X, sizeof(float) * (size_t)B * w->n_in, hipMemcpyHostToDevice, w->stream));
+    const pf::CopyPiece in{(void *)X, w->X, sizeof(float) * (size_t)B * w->n_in};
+    MHIP(w->slots.send(&in, 1, w->stream));
     MCHK(w->forward(B, w->X, nullptr));
     size_t ny = (size_t)B * w->n_out;
     k_denorm<<<(unsigned)((ny + 255) / 256), 256, 0, w->stream>>>(w->Yp, B, w->n_out, w->ym, w->ys, w->Yo);
     MHIP(hipGetLastError());
-    MHIP(hipMemcpyAsync(Y, w->Yo, sizeof(float) * ny, hipMemcpyDeviceToHost, w->stream));
-    MHIP(hipStreamSynchronize(w->stream));
+    const pf::CopyPiece out{Y, w->Yo, sizeof(float) * ny};
+    MHIP(w->slots.fetch(&out, 1, w->stream));
     return PF_OK;
 }
 
@@ -689,8 +690,8 @@ pf_status pf_warmstart_stage(pf_warmstart *w, const float *X, int B) {
     if (!w || !X || B <= 0 || B % 8) return PF_INVALID_ARG;
     MHIP(hipSetDevice(w->device));
     MCHK(w->ensure(B));
-    MHIP(hipMemcpyAsync(w->X, X, sizeof(float) * (size_t)B * w->n_in, hipMemcpyHostToDevice, w->stream));
-    MHIP(hipStreamSynchronize(w->stream));
+    const pf::CopyPiece in{(void *)X, w->X, sizeof(float) * (size_t)B * w->n_in};
+    MHIP(w->slots.send(&in, 1, w->stream));
     w->staged = B;
     return PF_OK;
 }
