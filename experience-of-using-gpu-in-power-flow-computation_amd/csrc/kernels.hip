@@ -230,11 +230,20 @@ __global__ void __launch_bounds__(256) k_head(DevNet N, DevState S, int lim, int
             atomicAdd(&ctl->flips, 1);
         mismatch_bus(N, S, k, P, Q, true, m, bad);
     }
+    // one atomic a block: 64 rows a block make 236 at 15,104 buses, and 944
+    // of them, one a wave, queued at the one address
+    __shared__ unsigned long long s_m[4];
+    __shared__ int s_bad[4];
     m = wave_max(m);
-    bad = __any(bad);
+    const int any_bad = __any(bad);
     if ((threadIdx.x & 63) == 0) {
-        atomicMax(&ctl->maxG_bits, double_as_u64(m));
-        if (bad) atomicOr(&ctl->simple_bad, 1u);
+        s_m[threadIdx.x >> 6] = double_as_u64(m);
+        s_bad[threadIdx.x >> 6] = any_bad;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        atomicMax(&ctl->maxG_bits, max(max(s_m[0], s_m[1]), max(s_m[2], s_m[3])));
+        if (s_bad[0] | s_bad[1] | s_bad[2] | s_bad[3]) atomicOr(&ctl->simple_bad, 1u);
     }
 }
 
