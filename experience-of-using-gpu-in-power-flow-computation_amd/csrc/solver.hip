@@ -19,6 +19,7 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -90,6 +91,7 @@ struct pf_solver {
     // theta, QliqLim, isq, limQ) with a pinned copy: one transfer either way
     char *state_dev = nullptr, *state_host = nullptr;
     size_t state_bytes = 0;
+    std::mutex state_mu;          // of state_host: threads may read a solver's state at once
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -383,6 +385,7 @@ pf_status pf_solver::set_isq_from_limq(const unsigned char *limQ) {
 // flat start (CPU/estrutura/barra.cpp:20-25 + PV/slack fields) and initLim
 // (CPU/limInjReat.cpp:177-207)
 pf_status pf_solver::reset_state() {
+    std::lock_guard<std::mutex> lk(state_mu);
     HIPCHK(hipStreamSynchronize(stream));   // an earlier copy may still read state_host
     const size_t nB = net.nB;
     double *h = (double *)state_host;
@@ -947,6 +950,7 @@ pf_status pf_solver_set_injections(pf_solver *s, const double *Pliq, const doubl
 pf_status pf_solver_get_state(pf_solver *s, double *V, double *theta, unsigned char *limQ) {
     if (!s) return PF_INVALID_ARG;
     HIPCHK(hipSetDevice(s->device));
+    std::lock_guard<std::mutex> lk(s->state_mu);
     PFCHK(s->get(s->state_host, (const char *)s->state_dev, s->state_bytes));
     const size_t nB = s->net.nB;
     const double *h = (const double *)s->state_host;

@@ -481,3 +481,24 @@ def test_nr_singular_with_a_pass_ahead(pf, cases, name, precision, metodo):
         r = s.solve()
         got.append([r[k] for k in ("status", "iterations", "converged", "singular")] + [x.tobytes() for x in s.state()])
     assert got[0] == got[1] and got[0][3]
+
+
+def test_state_read_by_several_threads(pf, cases):
+    """Threads that read one solver's state at once each get all of it."""
+    import threading
+    net = pf.Network(_path(cases, "c944"))
+    s = pf.Solver(net, pf.options(tolerancia=1e-8, no_max_iter=20))
+    s.solve(check=True)
+    want, got = s.state(), []
+
+    def read():
+        for _ in range(20):
+            got.append(s.state())
+
+    threads = [threading.Thread(target=read) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == 80
+    assert all(np.array_equal(x, y) for g in got for x, y in zip(want, g))
