@@ -1110,8 +1110,9 @@ __global__ void __launch_bounds__(256) k_residual(DevNet N, DevState S, int gate
 }
 
 // ----------------------------------------------------------------- update
+// A pass whose pivot failed has no step: the state stays as it was before.
 __global__ void __launch_bounds__(256) k_update(DevNet N, DevState S, int add_r, int gate) {
-    if (gate && !S.ctl->step) return;
+    if (gate && (!S.ctl->step || S.ctl->singular)) return;
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     double m = 0.0;
     if (k < N.nB && k != N.slack) {

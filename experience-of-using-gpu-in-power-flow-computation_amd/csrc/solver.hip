@@ -802,7 +802,7 @@ pf_status pf_solver::solve(pf_result *res) {
         const bool replay = opt.use_graph && path() == PF_ESPARSO;
         if (replay && !gexec) {
             HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-            pf_status st = enqueue_head(0);
+            pf_status st = enqueue_head(1);
             if (st == PF_OK) st = enqueue_step(1);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(stream, &g);
@@ -834,7 +834,6 @@ pf_status pf_solver::solve(pf_result *res) {
             if (c.done || c.singular) break;
         }
         HIPCHK(hipStreamSynchronize(stream));
-        if (replay) PFCHK(get(&c, ctl, 1));
     } else {
         if (trace_cb) {
             trace_lq.assign(net.nPV, 0);

@@ -146,7 +146,8 @@ typedef struct pf_result {
 pf_status pf_solver_create(const pf_network *net, const pf_options *opt, int device,
                            pf_solver **out);
 void pf_solver_destroy(pf_solver *s);
-/* NR from the current state (flat start after create / reset). */
+/* NR from the current state (flat start after create / reset).  PF_SINGULAR
+ * leaves the state that the failed pass started from: its step is not taken. */
 pf_status pf_solve(pf_solver *s, pf_result *res);
 pf_status pf_solver_reset(pf_solver *s);                 /* back to flat start */
 pf_status pf_solver_set_state(pf_solver *s, const double *V, const double *theta);

@@ -502,3 +502,25 @@ def test_state_read_by_several_threads(pf, cases):
         t.join()
     assert len(got) == 80
     assert all(np.array_equal(x, y) for g in got for x, y in zip(want, g))
+
+
+@pytest.mark.parametrize("name,precision,metodo", [("c14", "fp64", "ESPARSO"), ("c118", "mixed", "ESPARSO"),
+                                                   ("c944", "fp64", "ESPARSO"), ("c944", "mixed", "ESPARSO"),
+                                                   ("c118", "fp64", "DENSO"), ("c118", "fp64", "HIBRIDO_C")])
+def test_nr_singular_keeps_the_state(pf, cases, name, precision, metodo):
+    """A failed pivot ends the solve alike however its passes run (in one workgroup, launched one by one,
+    as a replayed graph, with stage timing): after the same pass, the state as it was before that step."""
+    net = pf.Network(_path(cases, name))
+    V0, th0 = np.zeros(net.nB), np.linspace(-0.1, 0.1, net.nB)
+    for graph in (0, 1):
+        for timing in (False, True):
+            s = pf.Solver(net, pf.options(tolerancia=1e-8, no_max_iter=10, use_graph=graph,
+                                          metodo=getattr(pf, metodo),
+                                          precision=pf.MIXED if precision == "mixed" else pf.FP64))
+            pf.lib().pf_solver_set_timing(s.h, int(timing))
+            s.set_state(V0, th0)
+            r = s.solve()
+            _say(name, precision, metodo, "graph", graph, "timing", timing, r)
+            assert (r["status"], r["iterations"], r["converged"], r["singular"]) == (pf.PF_SINGULAR, 1, False, True)
+            V, th, _ = s.state()
+            assert np.array_equal(V, V0) and np.array_equal(th, th0)
