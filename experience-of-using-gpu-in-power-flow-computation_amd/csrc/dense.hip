@@ -232,26 +232,31 @@ __global__ void __launch_bounds__(256) k_dense_update(double *A, double *b, int 
 }
 
 // U x = b from the last panel of 32 up.  Wave p % 8 solves panel p: lane i
-// holds its row i scaled to a unit diagonal, loaded since the wave's last
-// panel.  The threads above then subtract the panel's unknowns, their rows'
-// entries on it in registers by that time, so a panel waits for its 31
-// dependent multiply-adds and two barriers, not for loads.
+// holds its row i and its diagonal, loaded since the wave's last panel.  The
+// threads above then subtract the panel's unknowns, their rows' entries on it
+// in registers by that time, so a panel waits for its 32 dependent quotients
+// and multiply-adds and two barriers, not for loads.  A quotient is the
+// product with the diagonal's reciprocal, corrected by its remainder
+// (Markstein 1990: the rounded quotient, where nothing over- or underflows):
+// rows scaled by the reciprocal beforehand save two multiply-adds a step and
+// left 1 to 4 % more error.
 __global__ void __launch_bounds__(512) k_dense_back(const double *A, double *b, int n, Ctl *ctl, int gate) {
     if (gate && !ctl->step) return;
     if (ctl->singular) return;
     constexpr int NB = 32, NW = 8;
     __shared__ double s_y[kDenseMax], s_x[NB];
     const int tid = (int)threadIdx.x, lane = tid & 63, w = tid / 64, li = lane & (NB - 1);
-    double d[NB], rd = 0.0;   // this wave's coming panel: row li, and 1 / its diagonal
+    double d[NB], dg = 1.0, rd = 0.0;   // this wave's coming panel: row li, its diagonal and 1 / that
     auto diag = [&](int p) __attribute__((always_inline)) {
         if (p < 0) return;
         const int p0 = p * NB, nbc = min(NB, n - p0);
         const bool in = li < nbc;
-        rd = in ? 1.0 / (A + (size_t)p0 * n + p0)[(unsigned)li * (unsigned)(n + 1)] : 0.0;
+        dg = in ? (A + (size_t)p0 * n + p0)[(unsigned)li * (unsigned)(n + 1)] : 1.0;
+        rd = 1.0 / dg;
 #pragma unroll
         for (int j = 0; j < NB; j++) {
             const double x = (A + (size_t)(p0 + min(j, nbc - 1)) * n + p0)[(unsigned)min(li, nbc - 1)];
-            d[j] = in && j > li && j < nbc ? x * rd : 0.0;
+            d[j] = in && j > li && j < nbc ? x : 0.0;
         }
     };
     const int np = (n + NB - 1) / NB;
@@ -267,12 +272,20 @@ __global__ void __launch_bounds__(512) k_dense_back(const double *A, double *b, 
         }
         if (w == p % NW) {
             const bool in = li < nbc;
-            double y = in ? s_y[p0 + li] * rd : 0.0;
+            double y = in ? s_y[p0 + li] : 0.0, x = 0.0;
+            auto quotient = [&]() __attribute__((always_inline)) {
+                const double q = y * rd;
+                return fma(fma(-q, dg, y), rd, q);
+            };
 #pragma unroll
-            for (int j = NB - 1; j > 0; j--) y -= d[j] * lane_value(y, j);
+            for (int j = NB - 1; j >= 0; j--) {
+                const double q = quotient();
+                if (li == j) x = q;
+                y -= d[j] * lane_value(q, j);
+            }
             if (lane < NB) {   // zeros past the panel's columns
-                s_x[li] = y;
-                if (in) s_y[p0 + li] = y;
+                s_x[li] = x;
+                if (in) s_y[p0 + li] = x;
             }
             diag(p - NW);
         }
@@ -285,7 +298,7 @@ __global__ void __launch_bounds__(512) k_dense_back(const double *A, double *b, 
                 for (int j = 0; j < NB; j++) u[j] = (A + (size_t)(p0 + min(j, nbc - 1)) * n)[(unsigned)i];
             }
 #pragma unroll
-            for (int j = 0; j < NB; j++) y -= u[j] * s_x[j];
+            for (int j = NB - 1; j >= 0; j--) y -= u[j] * s_x[j];
             s_y[i] = y;
         }
         __syncthreads();
