@@ -1361,6 +1361,8 @@ struct pf_batch {
         for (hipEvent_t e : {ev_fork, ev_mid, ev_join, t0, t1})
             if (e) (void)hipEventDestroy(e);
         for (void *p : allocs) (void)hipFree(p);
+        for (auto &nb : nets)
+            if (nb->d_ws) (void)hipFree(nb->d_ws);
         for (auto s : st)
             if (s) (void)hipStreamDestroy(s);
     }
@@ -1635,7 +1637,8 @@ pf_status pf_batch::default_shape(BatchNet &nb, int nscen, int *block, int *per_
 }
 
 // launch shape of one topology: mode, workgroup size and workgroups per CU
-// (capped by occupancy); grows the global workspace when needed.
+// (capped by occupancy); a larger global workspace replaces the one before,
+// with the streams idle and the graph that names it dropped by the caller.
 pf_status pf_batch::configure(BatchNet &nb, int mode, int block, int per_cu) {
     auto refuse = [&](const char *why) {
         pf::set_last_error(std::string("batch launch shape (mode ") + std::to_string(mode) + ", block " +
@@ -1652,20 +1655,22 @@ pf_status pf_batch::configure(BatchNet &nb, int mode, int block, int per_cu) {
     BCHK(occupancy(nb, mode, block, &occ));
     if (occ < 1) return refuse("no workgroup fits on a CU (registers or LDS)");
     per_cu = per_cu <= 0 ? occ : std::min(per_cu, occ);
+    const int grid = std::max(1, std::min<int>((int)nb.scen.size(), per_cu * cus));
+    if (mode != 2) {   // before anything changes: on failure the shape stays as it was
+        const size_t need = (size_t)grid * (size_t)nb.ws;
+        if (need > nb.ws_cap) {
+            void *p = nullptr;
+            BHIP(hipMalloc(&p, need));
+            if (nb.d_ws) (void)hipFree(nb.d_ws);
+            nb.d_ws = (char *)p;
+            nb.ws_cap = need;
+        }
+    }
     nb.mode = mode;
     nb.block = block;
     nb.per_cu = per_cu;
     nb.shm = shm_bytes(nb, mode, block);
-    nb.grid = std::max(1, std::min<int>((int)nb.scen.size(), per_cu * cus));
-    if (mode != 2) {
-        const size_t need = (size_t)nb.grid * (size_t)nb.ws;
-        if (need > nb.ws_cap) {
-            char *p = nullptr;
-            BCHK(alloc(&p, need));
-            nb.d_ws = p;
-            nb.ws_cap = need;
-        }
-    }
+    nb.grid = grid;
     return PF_OK;
 }
 

@@ -1,6 +1,7 @@
 """GPU parity of the batched persistent solver (one workgroup per scenario)
 against the oracle solving each scenario on its own, and of its warm start /
 flat-start fallback.  Tolerance: |dV| <= 1e-6 pu, |dtheta| <= 1e-6 rad."""
+import ctypes
 import os
 import sys
 
@@ -451,3 +452,34 @@ def test_batch_long_row_pointers(pf, synth, tmp_path, precision):
     s.solve(check=True)
     V, th, _ = s.state()
     assert np.abs(outs[0][0][:nb] - V).max() <= 1e-9 and np.abs(outs[0][1][:nb] - th).max() <= 1e-9
+
+
+def _device_memory_free():
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_batch_shapes_hold_one_workspace(pf, synth, cases):
+    """A shape with more workgroups takes a larger workspace in place of the one before: from two to three
+    and from three to four slices a CU, memory grows by the one slice.  Same answers in each."""
+    net = pf.Network(cases.path("c944"))
+    n = 1024
+    P, Q, L = _scenarios(synth, net, n, 3900000)
+    b = pf.Batch([net], pf.options(tolerancia=1e-8, no_max_iter=8, precision=pf.MIXED))
+    b.set_scenarios(np.zeros(n, np.int32), P.ravel(), Q.ravel(), L.ravel())
+    grids, free, outs = [], [], []
+    for per_cu in (2, 3, 4):
+        b.set_shape(0, 1, 256, per_cu)
+        b.solve()
+        outs.append(b.results())
+        grids.append(b.shape(0)["grid"])
+        free.append(_device_memory_free())
+    _say("grids", grids, "free", free)
+    assert grids[1] - grids[0] == grids[2] - grids[1] > 0
+    d = np.diff(free)
+    assert d[0] < 0 and abs(d[1] / d[0] - 1) < 0.1
+    for o in outs[1:]:
+        for x, y in zip(outs[0], o):
+            assert np.array_equal(x, y, equal_nan=x.dtype.kind == "f")
