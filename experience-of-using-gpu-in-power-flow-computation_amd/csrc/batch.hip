@@ -1901,17 +1901,22 @@ pf_status pf_batch_solve(pf_batch *b, double *elapsed_ms) {
 // launch shape -- kernel MODE (working set in LDS / partly in LDS / global),
 // workgroup size, and for LDS topologies the resident workgroups per CU --
 // keep the fastest, and remember it in a text cache keyed by the device, the
-// topology's sizes, the numeric options and the scenario count, so later
-// runs apply it without measuring.
+// kernels' version, the topology's sizes, the numeric options and the scenario
+// count, so later runs apply it without measuring.
 }  // extern "C"
 
 namespace {
 
+// of k_batch's timing: goes up with a change that may move the fastest shape
+constexpr int kTuneVersion = 2;
+
 std::string tune_key(const pf_batch &b, const BatchNet &nb, const char *arch) {
     char k[512];
-    std::snprintf(k, sizeof k, "%s cus=%d nB=%d n=%d nnzL=%d nlev=%d nPV=%d prec=%d refine=%d lim=%d maxit=%d nscen=%zu",
-                  arch, b.cus, nb.net.nB, nb.sym.n, nb.sym.nnzL, nb.sym.nlev, nb.net.nPV, (int)b.opt.precision,
-                  b.opt.refine_steps, b.opt.lim_inj_reat ? 1 : 0, b.opt.no_max_iter, nb.scen.size());
+    std::snprintf(k, sizeof k,
+                  "%s kernels=%d cus=%d nB=%d n=%d nnzL=%d nlev=%d nPV=%d prec=%d refine=%d lim=%d maxit=%d nscen=%zu",
+                  arch, kTuneVersion, b.cus, nb.net.nB, nb.sym.n, nb.sym.nnzL, nb.sym.nlev, nb.net.nPV,
+                  (int)b.opt.precision, b.opt.refine_steps, b.opt.lim_inj_reat ? 1 : 0, b.opt.no_max_iter,
+                  nb.scen.size());
     return k;
 }
 

@@ -302,9 +302,9 @@ pf_status pf_batch_solve_noalloc(pf_batch *b, int n_scen, const int *net_of, con
  * metadata in LDS / all global; workgroup size; resident workgroups per CU),
  * keeps the fastest (minimum over `reps` timed launches after one warm-up)
  * and appends it to the text cache at cache_path (may be NULL: no cache).
- * A shape found in the cache for the same device, topology sizes, options and
- * scenario count is applied without measuring.  Outputs of the batch are
- * overwritten; call pf_batch_solve again afterwards.                        */
+ * A shape found in the cache for the same device, kernel version, topology
+ * sizes, options and scenario count is applied without measuring.  Outputs of
+ * the batch are overwritten; call pf_batch_solve again afterwards.          */
 pf_status pf_batch_autotune(pf_batch *b, const char *cache_path, int reps, int *n_measured);
 /* fix the launch shape of network `net` (after pf_batch_set_scenarios):
  * mode 2 needs the working set to fit in LDS, 1 the step vectors and level

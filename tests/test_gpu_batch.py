@@ -483,3 +483,24 @@ def test_batch_shapes_hold_one_workspace(pf, synth, cases):
     for o in outs[1:]:
         for x, y in zip(outs[0], o):
             assert np.array_equal(x, y, equal_nan=x.dtype.kind == "f")
+
+
+def test_batch_autotune_measures_for_its_own_kernels(pf, synth, cases, tmp_path):
+    """A cached shape was measured with one version of the kernels: an entry without a version, or with
+    another, is measured anew."""
+    net = pf.Network(cases.path("c944"))
+    P, Q, L = _scenarios(synth, net, 4, 3950000)
+    cache = tmp_path / "tune.txt"
+
+    def tune():
+        b = pf.Batch([net], pf.options(tolerancia=1e-8, no_max_iter=10, precision=pf.MIXED))
+        b.set_scenarios(np.zeros(4, np.int32), P.ravel(), Q.ravel(), L.ravel())
+        return b.autotune(str(cache), reps=1)
+
+    assert tune() >= 2 and tune() == 0
+    key, shape = cache.read_text().rstrip("\n").split("\t")
+    fields = key.split(" ")
+    version = [f for f in fields if f.startswith("kernels=")]
+    for other in ([], ["kernels=0"]):
+        cache.write_text(" ".join([f for f in fields if f not in version] + other) + "\t" + shape + "\n")
+        assert tune() >= 2
