@@ -702,7 +702,7 @@ __device__ __forceinline__ void wg_start(const BatchTopo &tp, Work<T> &w, const 
 // Returns (via shared result) iterations, converged flag, final max mismatch,
 // flips and whether a pivot failed (s_end, may be null).
 // s_chain: LDS of the dense top and of a narrow level's pivots; s_ck: of the
-// chunked narrow top, null: the working set is in LDS; rs, cl: row and column
+// chunked narrow top, null: level by level throughout; rs, cl: row and column
 // pointers of the flat sweeps.
 template <typename T, int TMAX, typename PTR>
 __device__ __forceinline__ void wg_nr(const BatchTopo &tp, const BatchJob &J, Work<T> &w, const double *Pliq,
@@ -955,18 +955,21 @@ struct LeanLds {
 // and barriers, which one workgroup alone does not cover: 2,048 x 944 buses in
 // FP32 9,840 us one of 1024, 7,090 two of 512; 2,048 x 354 buses 3,070 us two
 // of 256 at 183 VGPRs, 2,090 four at 128.
+// LEVELS: the level-by-level program of the sets in LDS, also where such a set
+// is asked to run in MODE 1 or 0 (one instantiation each, of 1024 threads), so
+// that a topology's answers do not depend on the placement.
 template <typename T, int MODE, int MAXT>
 constexpr int batch_min_waves() { return MODE == 1 ? 4 : (MODE == 2 && MAXT == 256 && sizeof(T) == 4) ? 3 : 1; }
 
-template <typename T, int MODE, int MAXT>   // MAXT: largest workgroup (register budget)
+template <typename T, int MODE, int MAXT, bool LEVELS = MODE == 2>   // MAXT: largest workgroup (register budget)
 __global__ void __launch_bounds__(MAXT, (batch_min_waves<T, MODE, MAXT>())) k_batch(BatchTopo tp0, BatchJob J) {
     extern __shared__ __align__(16) char smem[];
     __shared__ int s_item, s_it, s_conv, s_fl;
     constexpr bool lean = MODE == 1 && MAXT < 1024;                // its buffers are in smem (LeanLds)
     __shared__ B4<T> s_chain_own[lean ? 1 : 4 * batch_chain_cap<MODE>() + 2];   // dense top: row / column / pivot staging
-    __shared__ B4<T> s_ck_own[lean || MODE == 2 ? 1 : 2 * kBatchMaxChunks];     // chunk partial sums (a, u)
+    __shared__ B4<T> s_ck_own[lean || LEVELS ? 1 : 2 * kBatchMaxChunks];        // chunk partial sums (a, u)
     __shared__ double s_maxg;
-    B4<T> *s_chain = s_chain_own, *s_ck = MODE == 2 ? nullptr : s_ck_own;
+    B4<T> *s_chain = s_chain_own, *s_ck = LEVELS ? nullptr : s_ck_own;
     const int ck_max = lean ? tp0.ck_max : kBatchMaxChunks;
     BatchTopo tp = tp0;
     const DevNet &N = tp.N;
@@ -1182,8 +1185,8 @@ __global__ void k_zero_int(int *p, int n) {
     if (i < n) p[i] = 0;
 }
 
-// The instantiation for a precision, working-set placement and workgroup
-// size: compiled for at most 256, 512 or 1024 threads, so that smaller
+// The instantiation for a precision, working-set placement, workgroup size and
+// program (levels: of a set that fits in LDS): compiled for at most 256, 512 or 1024 threads, so that smaller
 // workgroups get the larger register budget.
 using BatchKernel = void (*)(BatchTopo, BatchJob);
 template <typename T, int MODE>
@@ -1192,7 +1195,9 @@ BatchKernel batch_kernel_t(int block) {
     if (block <= 512) return k_batch<T, MODE, 512>;
     return k_batch<T, MODE, 1024>;
 }
-inline BatchKernel batch_kernel(bool mixed, int mode, int block) {
+inline BatchKernel batch_kernel(bool mixed, int mode, int block, bool levels) {
+    if (levels && mode == 1) return mixed ? k_batch<float, 1, 1024, true> : k_batch<double, 1, 1024, true>;
+    if (levels && mode == 0) return mixed ? k_batch<float, 0, 1024, true> : k_batch<double, 0, 1024, true>;
     if (mixed)
         return mode == 2 ? batch_kernel_t<float, 2>(block)
                          : mode == 1 ? batch_kernel_t<float, 1>(block) : batch_kernel_t<float, 0>(block);
@@ -1238,6 +1243,8 @@ namespace {
 // set that leaves one workgroup per CU gains nothing: 236 buses in FP32
 // (80 KiB) 1,740 us in LDS, 1,140 us in MODE 1.
 constexpr long long kLdsLimit = 75 * 1024;
+// Sets up to here take no other placement; the larger ones do on request.
+constexpr long long kLdsOnly = 64 * 1024;
 }  // namespace
 
 // LDS bytes of k_solve_wg for a network, 0 where it does not run (the working
@@ -1528,30 +1535,27 @@ pf_status pf_batch::add_net(const pf_network &src) {
     b->lds = b->ws <= kLdsLimit;
     if (b->lds)
         for (int blk : {256, 512, 1024})
-            BHIP(hipFuncSetAttribute((const void *)batch_kernel(mixed, 2, blk),
+            BHIP(hipFuncSetAttribute((const void *)batch_kernel(mixed, 2, blk, true),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit));
     b->block = b->lds ? 256 : 1024;
     if (b->lds) {
         b->mode = 2;
         b->shm = b->ws;
-    } else {
+    }
+    if (b->ws > kLdsOnly) {
         long long pb = mixed ? partial_lds_bytes<float>(n, sym.nlev) : partial_lds_bytes<double>(n, sym.nlev);
         hipError_t e = hipSuccess;
         if (pb <= max_lds)
             for (int blk : {256, 512, 1024})
                 if (e == hipSuccess)
-                    e = hipFuncSetAttribute((const void *)batch_kernel(mixed, 1, blk),
+                    e = hipFuncSetAttribute((const void *)batch_kernel(mixed, 1, blk, b->lds),
                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            (int)(blk > 512 ? pb : max_lds));
-        if (pb <= max_lds && e == hipSuccess) {
-            b->partial = pb;
-            b->mode = 1;
-            b->shm = pb;
-        } else {
-            (void)hipGetLastError();
-            b->partial = 0;
-            b->mode = 0;
-            b->shm = 0;
+                                            (int)(blk > 512 || b->lds ? pb : max_lds));
+        if (e != hipSuccess) (void)hipGetLastError();
+        b->partial = pb <= max_lds && e == hipSuccess ? pb : 0;
+        if (!b->lds) {
+            b->mode = b->partial ? 1 : 0;
+            b->shm = b->partial;
         }
     }
     nets.push_back(std::move(b));
@@ -1561,7 +1565,7 @@ pf_status pf_batch::add_net(const pf_network &src) {
 // dynamic LDS of k_batch<T, mode> at this block size
 long long pf_batch::shm_bytes(const BatchNet &nb, int mode, int block) const {
     if (mode != 1) return mode == 2 ? nb.ws : 0;
-    if (block > 512) return nb.partial;
+    if (block > 512 || nb.lds) return nb.partial;
     const Symbolic &y = nb.sym;
     const int ck = nb.tp.ck_max;
     return opt.precision != PF_FP64 ? LeanLds<float>(y.n, y.nnzL, y.nlev, y.ch_m, ck).bytes
@@ -1578,7 +1582,7 @@ pf_status pf_batch::occupancy(BatchNet &nb, int mode, int block, int *per_cu) {
     const bool mixed = opt.precision != PF_FP64;
     const size_t shm = (size_t)shm_bytes(nb, mode, block);
     int pc = 0;
-    BHIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc, (const void *)batch_kernel(mixed, mode, block), block,
+    BHIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc, (const void *)batch_kernel(mixed, mode, block, nb.lds), block,
                                                       shm));
     *per_cu = known = pc;
     return PF_OK;
@@ -1646,8 +1650,8 @@ pf_status pf_batch::configure(BatchNet &nb, int mode, int block, int per_cu) {
         return PF_INVALID_ARG;
     };
     if (mode == 2 && !nb.lds) return refuse("the working set does not fit in LDS");
-    if (mode == 1 && (nb.lds || nb.partial == 0)) return refuse("mode 1 is for working sets beyond LDS whose step vectors fit");
-    if (mode == 0 && nb.lds) return refuse("the working set fits in LDS: use mode 2");
+    if (mode != 2 && nb.ws <= kLdsOnly) return refuse("a working set up to 64 KiB takes LDS only: use mode 2");
+    if (mode == 1 && nb.partial == 0) return refuse("mode 1 is for working sets whose step vectors fit in LDS");
     if (block < 64 || block > 1024 || block % 64) return refuse("block must be a multiple of 64 up to 1024");
     // the sweeps of modes 1 and 0 give each node of a narrow level its own 16 lanes
     if (mode != 2 && block < GL * kSweepGroupLevel) return refuse("modes 1 and 0 take at least 256 threads");
@@ -1699,7 +1703,7 @@ pf_status pf_batch::launch_net(size_t i, hipStream_t s) {
         const size_t shm = (size_t)b.shm;
         BatchTopo tp = b.tp;
         void *args[] = {&tp, &J};
-        BHIP(hipLaunchKernel((const void *)batch_kernel(mixed, b.mode, b.block), dim3(b.grid), dim3(b.block), args,
+        BHIP(hipLaunchKernel((const void *)batch_kernel(mixed, b.mode, b.block, b.lds), dim3(b.grid), dim3(b.block), args,
                              b.mode == 0 ? 0 : shm, s));
     }
     return PF_OK;
@@ -2163,7 +2167,7 @@ extern "C" pf_status pf_batch_solve_noalloc(pf_batch *b, int n_scen, const int *
         J.diverge = 1e6;
         BatchTopo tp = nb.tp;
         void *args[] = {&tp, &J};
-        BHIP(hipLaunchKernel((const void *)batch_kernel(mixed, nb.mode, plan[i].block), dim3(plan[i].grid),
+        BHIP(hipLaunchKernel((const void *)batch_kernel(mixed, nb.mode, plan[i].block, nb.lds), dim3(plan[i].grid),
                              dim3(plan[i].block), args, (size_t)b->shm_bytes(nb, nb.mode, plan[i].block), s));
     }
     if (!stream) {

@@ -504,3 +504,53 @@ def test_batch_autotune_measures_for_its_own_kernels(pf, synth, cases, tmp_path)
     for other in ([], ["kernels=0"]):
         cache.write_text(" ".join([f for f in fields if f not in version] + other) + "\t" + shape + "\n")
         assert tune() >= 2
+
+
+def _complete_graph(synth, nb, path):
+    rng = np.random.default_rng(nb)
+    buses = [synth.Bus(i + 1, 3 if i == 0 else 0, pload=round(float(rng.uniform(0, 2)), 1) * (i > 0),
+                       qload=round(float(rng.uniform(0, 0.5)), 1) * (i > 0)) for i in range(nb)]
+    branches = [synth.Branch(i + 1, j + 1, 1.0, round(float(rng.uniform(5, 9)), 3))
+                for i in range(nb) for j in range(i + 1, nb)]
+    synth.write_cdf(synth.Case(buses, branches), path)
+    return path
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_batch_placements_of_the_largest_lds_sets(pf, oracle, synth, cases, tmp_path, precision):
+    """Working sets of 64 to 75 KiB live in LDS by default and take the other two placements when asked,
+    with the same bits; the oracle's answers.  Sets up to 64 KiB take LDS only."""
+    path = os.path.join(GOLDEN, "c118.cdf") if precision == "fp64" else \
+        _complete_graph(synth, 45, str(tmp_path / "k45.cdf"))
+    net, n = pf.Network(path), 5
+    P, Q, L = _scenarios(synth, net, n, 3970000)
+    ref = _oracle_solve(oracle.Case(path), P, Q, L, lim=False)
+    for lu_blocked in (0, 1):
+        opts = pf.options(tolerancia=1e-8, no_max_iter=30, lu_blocked=lu_blocked,
+                          precision=pf.MIXED if precision == "mixed" else pf.FP64)
+        b = pf.Batch([net], opts)
+        b.set_scenarios(np.zeros(n, np.int32), P.ravel(), Q.ravel(), L.ravel())
+        _say(precision, lu_blocked, b.shape(0))
+        if lu_blocked:
+            assert b.shape(0)["mode"] == 2 and 64 * 1024 < b.shape(0)["lds_bytes"] <= 75 * 1024
+        if b.shape(0)["lds_bytes"] <= 64 * 1024:
+            continue
+        outs = []
+        for mode, block in ((2, 256), (1, 256), (1, 512), (1, 1024), (0, 256), (0, 512), (0, 1024)):
+            b.set_shape(0, mode, block)
+            assert b.shape(0)["mode"] == mode
+            b.solve()
+            outs.append(b.results() + (b.limq()[1],))
+        for o in outs[1:]:
+            for x, y in zip(outs[0], o):
+                assert np.array_equal(x, y)
+        for s, r in enumerate(ref):
+            k = slice(net.nB * s, net.nB * (s + 1))
+            assert outs[0][3][s] and r["converged"]
+            assert np.abs(outs[0][0][k] - r["V"]).max() <= 1e-6 and np.abs(outs[0][1][k] - r["theta"]).max() <= 1e-6
+    small = pf.Network(os.path.join(GOLDEN, "c14.cdf"))
+    b = pf.Batch([small], pf.options(tolerancia=1e-8, no_max_iter=30))
+    b.set_scenarios(np.zeros(1, np.int32), small.Pg - small.Pload, small.Qg - small.Qload, small.Qload)
+    for mode in (1, 0):
+        with pytest.raises(pf.PfError):
+            b.set_shape(0, mode, 256)
