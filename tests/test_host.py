@@ -310,3 +310,69 @@ def test_reader_pwf_known_answers(pf):
     ph = float(f32(-3.0)) * np.pi / 180
     assert np.array_equal(a["tap_re"], [1, 1, float(f32(0.978)) * np.cos(ph), 1, 1])
     assert np.array_equal(a["tap_im"], [0, 0, float(f32(0.978)) * np.sin(ph), 0, 0])
+
+
+def _plain_minimum_degree(n, edges):
+    """(blocks of L, levels of the elimination tree) of minimum degree, ties to the lower index."""
+    import heapq
+    adj = [set() for _ in range(n)]
+    for i, j in edges:
+        adj[i].add(j)
+        adj[j].add(i)
+    level, done, fill = [0] * n, [False] * n, 0
+    heap = [(len(a), i) for i, a in enumerate(adj)]
+    heapq.heapify(heap)
+    while heap:
+        d, v = heapq.heappop(heap)
+        if done[v] or d != len(adj[v]):
+            continue
+        done[v] = True
+        fill += d
+        for u in adj[v]:
+            adj[u] |= adj[v]
+            adj[u] -= {u, v}
+            level[u] = max(level[u], level[v] + 1)
+            heapq.heappush(heap, (len(adj[u]), u))
+    return fill, max(level) + 1
+
+
+def _probe_of_graph(pf, synth, path, nb, edges):
+    """The analysis of a network on these buses, 0 the slack, tied to bus 1 alone."""
+    buses = [synth.Bus(i + 1, 3 if i == 0 else 0) for i in range(nb + 1)]
+    branches = [synth.Branch(1, 2, 0.1, 1.0)] + [synth.Branch(i + 2, j + 2, 0.1, 1.0) for i, j in edges]
+    synth.write_cdf(synth.Case(buses, branches), path, wide=True)
+    return pf.SymbolicProbe(pf.Network(path))
+
+
+def test_order_of_a_radial_feeder(pf, synth, tmp_path):
+    """A feeder is a path with laterals: an order without fill takes it from one end, a level a bus.  The
+    order taken halves the path again and again: of 2,000 buses at most 4 log2 n levels, for at most
+    twice the blocks (a bus of a halved path has two neighbours left)."""
+    nb = 2000
+    edges = [(i, i + 1) for i in range(nb // 2 - 1)] + [(i, nb // 2 + i) for i in range(nb // 2)]
+    pr = _probe_of_graph(pf, synth, str(tmp_path / "radial.cdfx"), nb, edges)
+    fill, levels = _plain_minimum_degree(nb, edges)
+    assert fill == nb - 1
+    assert pr.nnzL <= 2 * nb and pr.levels <= 4 * np.log2(nb)
+    assert pr.levels < levels
+
+
+@pytest.mark.parametrize("kind", ["grid", "mesh"])
+def test_order_of_a_mesh(pf, synth, tmp_path, kind):
+    """Away from tied areas (a square grid; near neighbours of points in a square) the height in the key
+    costs at most a quarter more blocks of L than plain minimum degree, and no level."""
+    if kind == "grid":
+        m = 30
+        nb = m * m
+        edges = [(m * i + j, m * i + j + 1) for i in range(m) for j in range(m - 1)] + \
+                [(m * i + j, m * i + j + m) for i in range(m - 1) for j in range(m)]
+    else:
+        nb = 800
+        p = np.random.default_rng(9).random((nb, 2))
+        d = ((p[:, None] - p[None]) ** 2).sum(2)
+        near = np.argsort(d, 1)[:, 1:4]
+        edges = sorted({(min(i, int(j)), max(i, int(j))) for i in range(nb) for j in near[i]}
+                       | {(i, i + 1) for i in range(0, nb - 1, 40)})
+    pr = _probe_of_graph(pf, synth, str(tmp_path / "mesh.cdfx"), nb, edges)
+    fill, levels = _plain_minimum_degree(nb, edges)
+    assert pr.nnzL <= 1.25 * fill and pr.levels <= levels
