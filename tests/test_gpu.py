@@ -570,3 +570,29 @@ def test_dense_lu_solve_rounding(pf, cases, name):
     want = np.zeros(len(J))
     want[[at[i] for i in kept]] = [x[i] for i in kept]
     assert np.array_equal(s.lu_solve(V, th, None, b), want)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_lu_solve_longest_dense_top(pf, synth, tmp_path, precision):
+    """A complete graph of 120 buses: a dense top of 101 nodes in FP64 and 119 in FP32, past the 96 that
+    square tiles of the register inverse cover.  Accuracy as for the shorter ones."""
+    rng = np.random.default_rng(120)
+    nb = 120
+    buses = [synth.Bus(i + 1, 3 if i == 0 else 0, pload=round(float(rng.uniform(0, 2)), 1) * (i > 0),
+                       qload=round(float(rng.uniform(0, 0.5)), 1) * (i > 0)) for i in range(nb)]
+    branches = [synth.Branch(i + 1, j + 1, 1.0, round(float(rng.uniform(5, 9)), 3))
+                for i in range(nb) for j in range(i + 1, nb)]
+    path = str(tmp_path / "dense.cdf")
+    synth.write_cdf(synth.Case(buses, branches), path)
+    net = pf.Network(path)
+    assert pf.SymbolicProbe(net).chain[0] == 101
+    s = _solver(pf, net, precision=pf.MIXED if precision == "mixed" else pf.FP64)
+    V = 1.0 + 0.01 * np.random.default_rng(1).standard_normal(nb)
+    th = 0.05 * np.random.default_rng(2).standard_normal(nb)
+    rp, cj, v = s.jacobian(V, th, None)
+    n = len(rp) - 1
+    b = np.random.default_rng(4).standard_normal(n)
+    x = s.lu_solve(V, th, None, b)
+    r = np.zeros(n)
+    np.add.at(r, np.repeat(np.arange(n), np.diff(rp)), v * x[cj])
+    assert np.abs(r - b).max() <= 1e-9 * np.abs(v).max() * np.abs(x).max()

@@ -554,3 +554,36 @@ def test_batch_placements_of_the_largest_lds_sets(pf, oracle, synth, cases, tmp_
     for mode in (1, 0):
         with pytest.raises(pf.PfError):
             b.set_shape(0, mode, 256)
+
+
+@pytest.mark.parametrize("lu_blocked", [0, 1])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_batch_every_shape_beyond_lds(pf, oracle, synth, tmp_path, precision, lu_blocked):
+    """354 buses, beyond LDS in both precisions: every placement and workgroup size runs, with the same
+    bits, in both schedules; the oracle's answers."""
+    path = str(tmp_path / "c.cdfx")
+    synth.write_cdf(synth.multi_copy(3, 118000, 6, 3), path, wide=True)
+    net, n = pf.Network(path), 3
+    P, Q, L = _scenarios(synth, net, n, 3990000)
+    ref = _oracle_solve(oracle.Case(path), P, Q, L)
+    b = pf.Batch([net], pf.options(tolerancia=1e-8, no_max_iter=60, lim_inj_reat=1, lu_blocked=lu_blocked,
+                                   precision=pf.MIXED if precision == "mixed" else pf.FP64))
+    b.set_scenarios(np.zeros(n, np.int32), P.ravel(), Q.ravel(), L.ravel())
+    outs = []
+    for mode in (1, 0):
+        for block in (256, 512, 1024):
+            b.set_shape(0, mode, block)
+            _say("354 buses", precision, lu_blocked, b.shape(0))
+            assert (b.shape(0)["mode"], b.shape(0)["block"]) == (mode, block)
+            b.solve()
+            outs.append(b.results() + (np.concatenate(b.limq()[0]), b.limq()[1]))
+    for o in outs[1:]:
+        for x, y in zip(outs[0], o):
+            assert np.array_equal(x, y, equal_nan=x.dtype.kind == "f")
+    V, th, _, cv, _, lq, _ = outs[0]
+    for s, r in enumerate(ref):
+        k = slice(net.nB * s, net.nB * (s + 1))
+        assert bool(cv[s]) == bool(r["converged"])
+        if cv[s]:
+            assert np.abs(V[k] - r["V"]).max() <= 1e-6 and np.abs(th[k] - r["theta"]).max() <= 1e-6
+            assert np.array_equal(lq[net.nPV * s:net.nPV * (s + 1)], r["limQ"])
