@@ -248,3 +248,23 @@ def test_batch_results_in_parts(pf, synth, cases):
     for x, y in zip(every, own):
         assert np.array_equal(x, y.astype(x.dtype))
     assert len(np.unique(every[1].reshape(n, net.nB)[:, 5])) == n     # every scenario has angles of its own
+
+
+@pytest.mark.parametrize("rows", [40, 24])
+def test_fit_in_kept_room(pf, rows):
+    """A fit in the room that a larger one left, against the same fit in room of its own: 200 equal rows
+    once in batches of 40 and 40 of them five times are the same five steps, so both networks are at the
+    same weights and moments before it.  Same losses and weights, bit for bit."""
+    rng = np.random.default_rng(8)
+    x, y = rng.standard_normal((1, 16)).astype(np.float32), rng.standard_normal((1, 8)).astype(np.float32)
+    X, Y = rng.standard_normal((rows, 16)).astype(np.float32), rng.standard_normal((rows, 8)).astype(np.float32)
+    out = []
+    for n, epochs in ((200, 1), (40, 5)):
+        w = pf.WarmStart(16, 8, 24, 1, seed=3)
+        w.fit(np.repeat(x, n, 0), np.repeat(y, n, 0), epochs=epochs, batch=40)
+        before = w.params()
+        loss = w.fit(X, Y, epochs=2, batch=8)
+        out.append((before, np.asarray(loss), w.params()))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b) and np.all(np.isfinite(a))
+    assert not np.array_equal(out[0][0], out[0][2])
