@@ -598,7 +598,7 @@ pf_status pf_warmstart_grad(pf_warmstart *w, const float *X, const float *Y, int
 pf_status pf_warmstart_fit(pf_warmstart *w, const float *X, const float *Y, int n, int epochs, int B, float lr,
                            float weight_decay, unsigned long long seed, double *epoch_loss) {
     if (!w || !X || !Y || n < B || B <= 0 || B % 8 || epochs <= 0) return PF_INVALID_ARG;
-    w->staged = 0;   // the minibatches replace the staged rows
+    w->staged = 0;   // staged rows do not outlive a fit, whose batch size may take their room
     MHIP(hipSetDevice(w->device));
     MCHK(w->ensure(B));
     MCHK(w->fit_room(n));

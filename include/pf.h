@@ -166,7 +166,10 @@ pf_status pf_solver_lu_info(pf_solver *s, int *n, int *nnzL, int *levels, int *t
  * passes (P/Q, Jacobian, linear system with its refinement, state update),
  * the whole NR loop, and the last pf_solver_flows.  GPU phases are timed
  * with HIP events, so timing runs the NR loop with one host sync per pass
- * (use_graph is ignored while it is on).                                    */
+ * (use_graph is ignored while it is on).  A small network, whose loop one
+ * workgroup holds otherwise (tied 118-bus areas: up to 236 buses in FP64, 354
+ * mixed), takes the kernels across the GPU while timing or a trace is on: the
+ * same steps, summed in another order, so the last bits of V and theta differ. */
 typedef struct pf_timing {
     double ybus_ms, pq_ms, jacobian_ms, linear_ms, update_ms, iterative_ms, flows_ms;
     int passes;             /* NR passes timed (updates applied + the last check)  */
@@ -259,6 +262,8 @@ pf_status pf_probe_flat_factor_solve(const pf_symbolic_probe *p, double *blocks,
  * one workgroup owns one scenario for its whole NR solve.                   */
 typedef struct pf_batch pf_batch;
 
+/* a batch, like a warm start network, holds 4 MiB of pinned host memory for
+ * its transfers until it is destroyed                                       */
 pf_status pf_batch_create(const pf_network *const *nets, int n_nets, const pf_options *opt,
                           int device, pf_batch **out);
 void pf_batch_destroy(pf_batch *b);
@@ -337,7 +342,9 @@ pf_status pf_warmstart_set_params(pf_warmstart *w, const float *in);
 /* forward + backward of the mean squared error on normalised targets       */
 pf_status pf_warmstart_grad(pf_warmstart *w, const float *X, const float *Y, int B,
                             float *grads, double *loss);
-/* AdamW over a resident data set (n rows), minibatches of B (B % 8 == 0)   */
+/* AdamW over a resident data set (n rows), minibatches of B (B % 8 == 0).
+ * The rows' device memory stays with the network for the next fit, up to
+ * 256 MiB of it.                                                           */
 pf_status pf_warmstart_fit(pf_warmstart *w, const float *X, const float *Y, int n, int epochs,
                            int B, float lr, float weight_decay, unsigned long long seed,
                            double *epoch_loss);

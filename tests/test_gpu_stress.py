@@ -11,7 +11,7 @@ the others (the batch kernel stops a blown-up scenario early, the oracle runs
 it to the limit).
 The factors were chosen on the oracle: the last ones below the nose in steps
 of 0.01-0.05 (min |V| 0.55-0.67 pu there), and one past it.  At 15,104 buses
-the dense chain is a 202 x 202 FP32 Gauss-Jordan without pivoting; there the
+the dense chain is a 166 x 166 FP32 Gauss-Jordan without pivoting; there the
 flat-start Newton path is erratic near the nose (without Q limits 1.28-1.34
 diverge while 1.36-1.38 converge), and the test takes converging factors on
 both sides of that band and a diverging one inside it."""
